@@ -186,20 +186,21 @@ int dr_plan(int k, int m, int32_t* chunks, int32_t* kch, int32_t* rows_per_pass)
 /* What dr_matmul would launch for this launch, for inspection (replaces the plan dict that dense_reader/linear.py:
  * 455-495 choose/plan return): the kernel, the output tile width, the work split and the top-k records it writes. */
 typedef struct dr_launch_info {
-    int32_t kernel;        /* 0: the VALU GEMV (rows <= 2 a pass, and int4), 1: the MFMA kernel */
-    int32_t rows_per_pass;
+    int32_t kernel;        /* 0: the VALU GEMV (rows <= 2 a pass, and int4), 1: an MFMA kernel */
+    int32_t rows_per_pass; /* (from 129 rows on one launch takes all rows: its workgroups' rows, 64 to 256) */
     int32_t tile_cols;     /* output columns of a work tile: 16 (one panel) or 32 */
     int32_t tiles;         /* work tiles of the launch */
     int32_t chunks;        /* K chunks a tile, kch values each */
     int32_t kch;
     int32_t splits;        /* workgroups a tile (split K), 1 if unsplit */
     int32_t workgroups;    /* workgroups of one pass */
-    int32_t passes;        /* launches (row passes) */
+    int32_t passes;        /* row passes: launches, or (from 129 rows on) the row tiles of the one launch */
     int32_t records;       /* top-k records the launch writes (0: no top-k) */
     int32_t tiles_per_record;
     int32_t waves;         /* wavefronts a workgroup (each walks its K chunks in turn) */
     int32_t tiles_per_workgroup; /* 2: a 32-row launch of more tiles than CUs, its block-float segments' tiles in
-                                    pairs (bf16 segments one a workgroup), else 1 */
+                                    pairs (bf16 segments one a workgroup); from 129 rows on 8 or 2 (a GLU's 4 or 1);
+                                    else 1 */
     int32_t lds_bytes;     /* LDS a workgroup of the first pass's kernel, static and dynamic (0 without a device) */
     int32_t reserved[2];
 } dr_launch_info;

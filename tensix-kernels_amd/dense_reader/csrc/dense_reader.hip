@@ -31,22 +31,22 @@
 
 #include "dense_reader.h"
 #include "moe.h"
+#include "dense_gemm.h"
+#include "dr_device.h"
 #include "../../moe/csrc/moe_route.h"
 #include "wave_select.h"
 
-// No contraction of a multiply and an add into an FMA unless the code asks for one: the compiler would otherwise
-// decide per kernel instantiation, and a weight would round differently in a block list than alone.
 #pragma clang fp contract(off)
 
 namespace {
 
-constexpr int KALIGN = 256;  // K padding: one exponent group; a multiple of every format's k-block
+using namespace drk;
+
 constexpr int MAXW = 8;      // wavefronts a workgroup at most (512 threads: up to 256 VGPRs a lane)
 // The expert-gathered GEMV's down modes: up to 16 wavefronts (1024 threads; those kernels stay under 128 VGPRs). A
 // CU's bytes follow the chunks it has in flight: the gpt-oss down (180 workgroups of 24 chunks) 8.0 -> 6.9 us with 16
 // wavefronts of one or two chunks against 8 of three (12 of two: 7.5 us).
 constexpr int MAXW_DOWN = 16;
-constexpr int TILE = 32;
 
 // output columns of a workgroup's tile: 16 (one panel) for a narrow launch (PW = 1), else 32
 template <int PW>
@@ -54,9 +54,6 @@ __host__ __device__ constexpr int tile_w() {
     return PW == 1 ? 16 : TILE;
 }
 
-__host__ __device__ constexpr int kblk(int fmt) {
-    return fmt == DR_BFP8 ? 64 : (fmt == DR_BFP4 || fmt == DR_INT4 || fmt == DR_BFP4_KB) ? 128 : 32;
-}
 
 // DR_BFP4_KB: the byte of a panel's exponents that holds column c's exponent for k (one a 16-k group): per 128-k block
 // 128 bytes, lane (kq, c) of the block's wavefront load at 2 (16 kq + c), its two groups (k 32 kq + 0..15, + 16..31)
@@ -74,31 +71,10 @@ __host__ __device__ constexpr int exp_off(int fmt, int k) {
 
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 
-__device__ __forceinline__ float bf16_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
-
-// fp32 -> bf16 bits, round to nearest even; a NaN becomes the quiet NaN 0x7FC0
-__device__ __forceinline__ uint32_t f32_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7FFFFFFFu) > 0x7F800000u) return 0x7FC0u;
-    return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
-}
-
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
 }
 
-struct SegDev {
-    const uint8_t* codes;
-    const uint8_t* exps;
-    const uint8_t* codes_up;
-    const uint8_t* exps_up;
-    const void* scale;
-    const void* scale_up;
-    const uint16_t* gscale;  // DR_INT4: the group scales [panel][k-block][4][16] bf16
-    int fmt, n, n_pad, glu, scale_f32, col0;
-    int n_out, tiles, tile_begin;
-    unsigned pstride;  // bytes of codes a panel
-};
 
 struct Args {
     const uint16_t* x;
@@ -718,10 +694,6 @@ __device__ __forceinline__ void chunk_bf16(const Args& a, const uint8_t* const* 
     }
 }
 
-__device__ __forceinline__ float load_scale(const void* s, int f32, int col) {
-    if (s == nullptr) return 1.f;
-    return f32 ? reinterpret_cast<const float*>(s)[col] : bf16_to_f32(reinterpret_cast<const uint16_t*>(s)[col]);
-}
 
 // The epilogue's operands from memory (column scales, residual), read before the K loop so that their latency hides
 // under it instead of adding to the workgroup's end: thread c < TW (the tile's width) the scales of the tile's output
@@ -773,12 +745,6 @@ __device__ __forceinline__ void epi_stage(const EpiPre& p, float* pre) {
     pre[PRE_RES + e] = p.res;
 }
 
-// the dense GLU's activation: silu(g) = g * sigmoid(g); gelu_tanh(g) = g * sigmoid(1.5957691216 g + 0.0713548162 g^3)
-// (dense_ops.h:46-59)
-__device__ __forceinline__ float act_glu(float g, int act) {
-    const float z = act == DR_ACT_GELU_TANH ? g * (1.5957691216f + 0.0713548162f * (g * g)) : g;
-    return g / (1.f + __expf(-z));
-}
 
 // the experts' act(g) * u: act_glu's two, or swiglu_oai min(g, 7) * sigmoid(1.702 min(g, 7)) * (clamp(u, -7, 7) + 1)
 // (dense_ops.h:90-118), a NaN passing through the clamps as it does there (the dense GLU keeps act_glu alone: the
@@ -1532,8 +1498,6 @@ dr_gemv_moe(const MoeArgs a) {
 // block-float m * 2^(E - bias) (exact in bf16: at most 7 significant bits), the power of two broadcast across the row
 // from the lane that read that k's exponent. Output lane l: rows 4 (l / 16) .. +3 of column l % 16.
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 // d = broadcast(s from lane I of this row of 16) * f (the same hazard rule as fmac_bcast)
 template <int I, bool NOP>
@@ -1548,10 +1512,6 @@ __device__ __forceinline__ float mul_bcast(float s, float f) {
     return d;
 }
 
-// two fp32 values with at most 8 significant bits as one bf16 pair (truncation is exact)
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
 
 // 16 bytes of x: row m, columns k .. k + 7 (k a multiple of 8). Rows past x read its last row: they only reach output
 // rows that are never written. Columns past K read its last columns and are zeroed by x_kmask (the weights there are
@@ -1621,9 +1581,6 @@ __device__ __forceinline__ uint4 x_lds(const uint4* xs, int row, int c) {
     return xs[NCH * row + (c ^ x_swz<NCH>(row))];
 }
 
-__device__ __forceinline__ f32x4 mfma(uint4 a, uint4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
 
 // B for 8 bfp8 values: bytes 8H .. 8H + 7 of the lane's codes (k-offsets 16 kq + 8H + j), times the broadcast scales
 template <int H>
@@ -3314,6 +3271,63 @@ void bind_split(Args& a, void* workspace, int pw, int mr) {
     if (a.rec != nullptr && a.tk_group > 1) a.rec_out = a.tstage;
 }
 
+// ---- many rows: the tiled kernel (dense_gemm.hip) -----------------------------------------------------------------------
+//
+// From GEMM_MIN_M rows on, one weight without top-k records runs as one launch of dr_gemm instead of passes of 32 rows,
+// each of which reads and decodes every weight again. Against the passes on MI355X at 129, 256 and 1024 rows: bfloat8_b
+// K = 4096 N = 14336 70, 114, 449 -> 50, 51, 113 us; K = 14336 N = 4096 104, 165, 648 -> 60, 63, 172; K = 1024 N = 1024
+// 37, 44, 180 -> 14 (the call's host time). Up to 128 rows the passes stay: their rows equal those of a call on them
+// alone bit for bit.
+constexpr int GEMM_MIN_M = 129;
+
+// The tile: mt row tiles of 32 with the wavefronts side by side (256 columns a workgroup, 128 with a GLU), or ks, 64
+// rows x 64 columns with the wavefronts splitting K. The one of the least time by rounds of workgroups over the CUs
+// (one workgroup a CU) x (start and end + 64-k steps x the step's time), in units of 10 ns as measured at K = 4096 and
+// 14336 (one round of each: 64 rows 48 and 154 us, 128 rows 62 and 199, 192 rows 80 and 258, 256 rows 100 and 322, ks 17
+// and 60).
+struct GemmTile {
+    int mt;
+    bool ks;
+    int start, step;
+};
+constexpr GemmTile GEMM_TILES[] = {{2, true, 100, 28}, {2, false, 300, 66}, {4, false, 500, 86}, {6, false, 700, 111}, {8, false, 900, 139}};
+
+// false: the launch runs in passes
+bool gemm_plan(const dr_launch* L, const Args& a, GemmArgs& g, GemmTile& best) {
+    if (L->m < GEMM_MIN_M || a.nseg != 1 || a.rec != nullptr || a.seg[0].fmt > DR_BF16) return false;
+    const SegDev& s = a.seg[0];
+    g = GemmArgs{};
+    g.x = a.x;
+    g.m = a.m;
+    g.k = a.k;
+    g.k_pad = a.k_pad;
+    g.ldx = a.ldx;
+    g.y = a.y;
+    g.ldy = a.ldy;
+    g.y_f32 = a.y_f32;
+    g.res = a.res;
+    g.ldr = a.ldr;
+    g.res_mode = a.res_mode;
+    g.act = a.act;
+    g.seg = s;
+    g.tiles = (s.n_out + TILE - 1) / TILE;
+    g.vec4 = a.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(a.y) % (a.y_f32 ? 16 : 8) == 0;
+    long long least = -1;
+    for (const GemmTile& t : GEMM_TILES) {
+        const int per = (s.glu ? 1 : 2) * (t.ks ? 1 : GEMM_W);  // output tiles a workgroup
+        const long long tm = (a.m + 32 * t.mt - 1) / (32 * t.mt), tn = (g.tiles + per - 1) / per;
+        const long long rounds = (tm * tn + cu_count() - 1) / cu_count();
+        const long long cost = rounds * (t.start + (long long)(a.k_pad / 64) * t.step);
+        if (tm * tn > INT32_MAX || (least >= 0 && cost >= least)) continue;
+        least = cost;
+        best = t;
+        g.tm = (int)tm;
+        g.tn = (int)tn;
+    }
+    // (a tile's rows of x lie within the buffer loads' 31-bit offsets)
+    return least >= 0 && (int64_t)a.ldx * 2 * 256 < INT32_MAX;
+}
+
 // dr_matmul's launches: one pass of up to mr rows each (the passes a top-k launch needs, not y, skipped)
 int run_passes(const dr_launch* L, const Args& a, int tiles, int mr, int pw, hipStream_t st) {
     const size_t ysz = a.y_f32 ? 4 : 2;
@@ -3424,6 +3438,9 @@ int64_t dr_workspace_bytes(const dr_launch* L) {
     int pw, tiles, mr;
     if (L != nullptr && L->act == DR_ACT_SWIGLU_OAI) return -1;  // (the dense GLU: silu or gelu_tanh)
     if (prepare(L, a, pw, tiles, mr) != DR_OK) return -1;
+    GemmArgs g;
+    GemmTile gt;
+    if (gemm_plan(L, a, g, gt)) return 0;
     return workspace_bytes(a, pw, mr);
 }
 
@@ -3433,6 +3450,9 @@ int dr_matmul(const dr_launch* L) {
     if (L != nullptr && L->act == DR_ACT_SWIGLU_OAI) return DR_EINVAL;  // (the dense GLU: silu or gelu_tanh)
     const int st0 = prepare(L, a, pw, tiles, mr);
     if (st0 != DR_OK) return st0;
+    GemmArgs g;
+    GemmTile gt;
+    if (gemm_plan(L, a, g, gt)) return hip_status(launch_gemm(g, gt.mt, gt.ks, S(L->stream)));
     const int64_t need = workspace_bytes(a, pw, mr);
     if (need > 0) {
         // split K needs the workspace: its counters start at zero (the caller zeroes it once; each launch leaves
@@ -3460,6 +3480,9 @@ int dr_matmul_noalloc(const dr_launch* L) {
     if (L != nullptr && L->act == DR_ACT_SWIGLU_OAI) return DR_EINVAL;
     const int st0 = prepare(L, a, pw, tiles, mr);
     if (st0 != DR_OK) return st0;
+    GemmArgs g;
+    GemmTile gt;
+    if (gemm_plan(L, a, g, gt)) return hip_status(launch_gemm(g, gt.mt, gt.ks, S(L->stream)));
     const int64_t need = workspace_bytes(a, pw, mr);
     if (need > DR_SCRATCH_BYTES) return DR_ERANGE;  // (checked before any device call)
     hipStream_t st = S(L->stream);
@@ -3480,6 +3503,23 @@ int dr_launch_plan(const dr_launch* L, dr_launch_info* info) {
     const int st = prepare(L, a, pw, tiles, mr);
     if (st != DR_OK) return st;
     *info = dr_launch_info{};
+    GemmArgs g;
+    GemmTile gt;
+    if (gemm_plan(L, a, g, gt)) {
+        info->kernel = 1;
+        info->rows_per_pass = 32 * gt.mt;
+        info->tile_cols = TILE;
+        info->tiles = g.tiles;
+        info->chunks = 1;
+        info->kch = a.k_pad;
+        info->splits = 1;
+        info->workgroups = g.tn;
+        info->tiles_per_workgroup = (a.seg[0].glu ? 1 : 2) * (gt.ks ? 1 : GEMM_W);
+        info->passes = g.tm;
+        info->waves = GEMM_W;
+        info->lds_bytes = (int32_t)gemm_lds(gt.mt, gt.ks);
+        return DR_OK;
+    }
     info->kernel = (mr >= 16) ? 1 : 0;
     info->rows_per_pass = mr;
     info->tile_cols = pw == 1 ? 16 : TILE;
@@ -3515,6 +3555,21 @@ int dr_launch_work(const dr_launch* L, int32_t* work, int max_workgroups) {
     if (L != nullptr && L->act == DR_ACT_SWIGLU_OAI) return DR_EINVAL;
     const int st = prepare(L, a, pw, tiles, mr);
     if (st != DR_OK) return st;
+    GemmArgs gm;
+    GemmTile gt;
+    if (gemm_plan(L, a, gm, gt)) {  // (a row tile's workgroups, one a column tile)
+        if (gm.tn > max_workgroups) return DR_ERANGE;
+        const int per = (a.seg[0].glu ? 1 : 2) * (gt.ks ? 1 : GEMM_W);
+        for (int i = 0; i < gm.tn; ++i) {
+            int32_t* o = work + 5 * (size_t)i;
+            o[0] = 0;
+            o[1] = i * per;
+            o[2] = min(per, gm.tiles - i * per);
+            o[3] = 0;
+            o[4] = a.seg[0].col0 + i * per * TILE;
+        }
+        return DR_OK;
+    }
     const int wgs = a.pairs > 0 ? a.pairs : tiles * a.splits;
     if (wgs > max_workgroups) return DR_ERANGE;
     const int cols = pw == 1 ? 16 : TILE;

@@ -282,8 +282,8 @@ def reference(x, w, scale=None):
 
 def row_slices(x, full_sync=False):
     """[(first tile row, tile rows)] of x's rows, at most 4 tile rows each (8 with full_sync) (reference linear.py:
-    179-184, where each slice is one program that reads all the weights). matmul needs no slicing: one launch takes
-    all of x's rows, in passes of plan()["rows_per_pass"] inside it. A caller that slices x this way gets each slice's
+    179-184, where each slice is one program that reads all the weights). matmul needs no slicing: one call takes all of
+    x's rows, up to 128 of them in passes of plan()["rows_per_pass"], more in one launch of a tiled kernel. A caller that slices x this way gets each slice's
     rows from its own matmul (the rows a call takes pick its kernel, so the sums of a slice's rows can differ in their
     last bits from those of one call over all rows)."""
     mt = -(-x.shape[-2] // TILE)

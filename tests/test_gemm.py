@@ -1,0 +1,167 @@
+"""The matmul of many rows (dense_gemm.hip): every tile of its plan, each format, at the edges of its tiles, against the
+CPU oracle; and the order of its staging in the emitted code.
+
+Bars as for the other kernels (the reference's): 1 % relative Frobenius error and PCC 0.9999 for bf16 outputs, 0.1 % for
+fp32 outputs. Every row is its own MFMA column, summed in an order that depends on K and the tile only, so permuting x's
+rows permutes y's bit for bit and repeated calls agree.
+"""
+
+import re
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+import torch
+
+from common.testing import check, same
+from dense_reader import linear
+from oracle import dense_oracle as O
+
+FMTS = {"bfp8": linear.bfloat8_b, "bfp4": linear.bfloat4_b, "bf16": linear.bfloat16}
+
+
+def _x(dev, m, k, seed):
+    x = O.x_input(m, k, seed)
+    return x, x.to(torch.bfloat16).reshape(1, 1, m, k).to(dev.torch)
+
+
+def _weight(dev, n, k, fmt, seed):
+    wt = O.matrix(n, k, seed)
+    return linear.native_weight(dev, wt, FMTS[fmt])[0], torch.from_numpy(O.held(wt.T.contiguous(), fmt))
+
+
+def _host(y, m):
+    return y.float().cpu().reshape(m, -1)
+
+
+# (rows, K, N, rows a tile, output tiles a workgroup): every tile of the plan; rows past the last tile, K off the
+# 256-k group and off the 64-k step, N off the tile, the workgroup's columns and the 4-column store
+SHAPES = [
+    (129, 96, 40, 64, 2),
+    (160, 800, 545, 64, 2),  # the wavefronts split K: groups of 256 k unevenly
+    (257, 4352, 96, 64, 2),
+    (130, 288, 14340, 64, 8),
+    (192, 512, 32768, 128, 8),
+    (160, 512, 65537, 192, 8),
+    (1023, 256, 16382, 256, 8),
+    (1000, 800, 14336, 256, 8),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", list(FMTS))
+@pytest.mark.parametrize("m, k, n, rows, tiles", SHAPES)
+def test_tiles(device, fmt, m, k, n, rows, tiles):
+    tw, h = _weight(device, n, k, fmt, 1)
+    x, tx = _x(device, m, k, 2)
+    p = linear.launch_plan(tx, tw, None)
+    print(p, flush=True)
+    assert (p["kernel"], p["rows_per_pass"], p["tiles_per_workgroup"]) == ("mfma", rows, tiles), p
+    assert p["passes"] == -(-m // rows) and p["workgroups"] == -(-p["tiles"] // tiles)
+    s = torch.rand(n, generator=torch.Generator().manual_seed(3)) + 0.5
+    ts = linear.scale_tensor(device, s, dtype=linear.float32)
+    y = _host(linear.matmul(tx, tw, ts), m)
+    check(f"{fmt} rows {m} K {k} N {n} scaled", y, O.ref(x, h, s))
+    same("repeated call", _host(linear.matmul(tx, tw, ts), m), y)
+    perm = torch.randperm(m, generator=torch.Generator().manual_seed(4))
+    yp = _host(linear.matmul(tx[..., perm.to(tx.device), :].contiguous(), tw, ts), m)
+    same("rows permuted", yp, y[perm])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", list(FMTS))
+@pytest.mark.parametrize("m, k, n", [(131, 800, 200), (200, 288, 14340)])
+def test_epilogue(device, fmt, m, k, n):
+    """Residual (both modes, bf16 and fp32 outputs, in place), fp32 output, col0 into a wider output."""
+    tw, h = _weight(device, n, k, fmt, 11)
+    x, tx = _x(device, m, k, 12)
+    want = O.ref(x, h)
+    res = torch.randn(m, n, generator=torch.Generator().manual_seed(13)).to(torch.bfloat16)
+    tr = res.reshape(1, 1, m, n).to(device.torch)
+    for mode in ("epilogue", "preload"):
+        y = _host(linear.matmul(tx, tw, None, residual=tr, residual_mode=mode), m)
+        check(f"residual {mode}", y, want + res.float())
+        y = _host(linear.matmul(tx, tw, None, residual=tr, residual_mode=mode, out32=True), m)
+        check(f"residual {mode} fp32", y, want + res.float(), rel=1e-3, pcc=0.999999)
+    inplace = tr.clone()
+    assert linear.matmul(tx, tw, None, residual=inplace, out=inplace) is inplace
+    check("residual in place", _host(inplace, m), want + res.float())
+    check("fp32 output", _host(linear.matmul(tx, tw, None, out32=True), m), want, rel=1e-3, pcc=0.999999)
+    wide = torch.full((1, 1, m, 32 + n + 32), 7.0, dtype=torch.bfloat16, device=device.torch)
+    linear.matmul(tx, tw, None, out=wide, col0=1)
+    y = _host(wide, m)
+    check("col0", y[:, 32:32 + n], want)
+    rest = torch.cat([y[:, :32], y[:, 32 + n:]], 1)
+    same("the other columns untouched", rest, torch.full_like(rest, 7.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", list(FMTS))
+@pytest.mark.parametrize("m, k, n", [(129, 800, 96), (150, 256, 7200), (333, 288, 8224), (600, 96, 8192)])
+def test_glu(device, fmt, m, k, n):
+    """Gate and up apart (with column scales) and interleaved, silu and gelu_tanh."""
+    gw, uw = O.matrix(n, k, 21), O.matrix(n, k, 22)
+    hg, hu = (torch.from_numpy(O.held(w.T.contiguous(), fmt)).float() for w in (gw, uw))
+    tg, tu, ti = (linear.native_weight(device, w, FMTS[fmt])[0] for w in (gw, uw, linear.interleave_glu(gw, uw)))
+    x, tx = _x(device, m, k, 23)
+    s = torch.rand(2, n, generator=torch.Generator().manual_seed(24)) + 0.5
+    tsg, tsu = (linear.scale_tensor(device, v, dtype=linear.float32) for v in s)
+    tsi = linear.scale_tensor(device, torch.stack([s[0].reshape(-1, 32), s[1].reshape(-1, 32)], 1).reshape(-1),
+                              dtype=linear.float32)
+    xd = x.to(torch.bfloat16).double()
+    g, u = (xd @ hg.double()) * s[0].double(), (xd @ hu.double()) * s[1].double()
+    for act, code in (("swiglu", 0), ("geglu", 1)):
+        two = _host(linear.matmul(tx, tg, tsg, glu=True, w_up=tu, scale_up=tsu, glu_act=code), m)
+        check(f"{fmt} {act} two weights", two, O.glu_ref(g, u, act))
+        same("interleaved against two weights", _host(linear.matmul(tx, ti, tsi, glu=True, glu_act=code), m), two)
+
+
+@pytest.mark.gpu
+def test_columns_past_k_and_nan(device):
+    """A ragged K: what lies past K in x's memory (the next row, here Inf and NaN) enters no sum; a NaN row stays its
+    own row's."""
+    m, k, n = 140, 288, 64
+    tw, h = _weight(device, n, k, "bfp8", 31)
+    x, _ = _x(device, m, k, 32)
+    x[5] = float("nan")
+    x[7, 3] = float("inf")
+    y = _host(linear.matmul(x.to(torch.bfloat16).reshape(1, 1, m, k).to(device.torch), tw, None), m)
+    assert bool(y[5].isnan().all()) and not bool(y[7].isfinite().any())
+    keep = [r for r in range(m) if r not in (5, 7)]
+    check("the other rows", y[keep], O.ref(x[keep], h))
+
+
+def test_staging_order():
+    """In the emitted gfx950 code of dr_gemm every barrier of the K loop follows a wait for the wavefront's LDS reads
+    (lgkmcnt(0)) and for all but its newest x loads (vmcnt of at most two stages), and between two such barriers lie one
+    stage's loads to LDS, so that a stage is read only after its loads have landed and overwritten only after its reads."""
+    import __graft_entry__ as G
+
+    hipcc = G.HIPCC if Path(G.HIPCC).exists() else shutil.which("hipcc")
+    if hipcc is None:
+        pytest.skip("no hipcc")
+    src = next(s for s in G.SOURCES if s.stem == "dense_gemm")
+    flags = [f for f in G.FLAGS if f not in ("-shared", "-fPIC")]
+    r = subprocess.run([hipcc, *flags, "--cuda-device-only", "-S", str(src), "-o", "-"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    found = 0
+    for name, body in re.findall(r"^(_ZN3drk\S*dr_gemmI\S*):(.*?)s_endpgm", r.stdout, re.M | re.S):
+        mt, ks = (int(v) for v in re.search(r"dr_gemmILi(\d+)ELi\dELb\dELb(\d)E", name).groups())
+        stage = 4 * mt if ks else mt  # loads to LDS a stage, of one wavefront
+        lines = [s.strip() for s in body.split("\n")]
+        lines = [s for s in lines if s and not s.startswith((";", ".")) and not s.endswith(":")]
+        dma = [i for i, s in enumerate(lines) if s.startswith("buffer_load") and s.endswith("lds")]
+        waits = [(i, int(m.group(1))) for i, s in enumerate(lines)
+                 if (m := re.match(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)", s)) and int(m.group(1)) in (stage, 2 * stage)]
+        inside = [i for i, v in waits if v == stage]
+        # three stages asked for ahead of the loop, then one after each of its waits (four steps a turn)
+        assert len(inside) >= 4 and len(inside) % 4 == 0 and len(dma) == (3 + len(inside)) * stage, (name, len(dma))
+        assert [v for _, v in waits if v != stage] == [2 * stage] and sum(i < inside[0] for i in dma) == 3 * stage
+        for a, b in zip(inside, inside[1:] + [len(lines)]):
+            if not ks:
+                nxt = next(s for s in lines[a + 1:] if not s.startswith("s_waitcnt"))
+                assert nxt == "s_barrier", (name, lines[a], nxt)
+            assert sum(a < i < b for i in dma) == stage, (name, a, b)
+        found += 1
+    assert found == 30, found
