@@ -151,7 +151,8 @@ typedef struct dr_launch {
 int64_t dr_workspace_bytes(const dr_launch* launch);
 
 /* y = the launch's fused matmul. Allocates nothing. A DR_INT4 weight goes alone (one segment, no GLU, residual or
- * top-k) and takes its rows two at a time (int4/w4a16.py:170-253 w4a16_linear takes one token). */
+ * top-k); up to 5 rows on the GEMV (each row's result that of a one-row call), more on the MFMA kernel
+ * (int4/w4a16.py:170-253 w4a16_linear takes one token). */
 int dr_matmul(const dr_launch* launch);
 
 /* dr_matmul without a caller workspace: a launch that needs one (dr_workspace_bytes > 0) uses the library's own,
@@ -179,14 +180,14 @@ int dr_topk_merge(const void* records, int n_records, int rows, int k, int fp32,
 
 /* The work split for K and M: chunks (waves per output tile, each a K range of kch values) and the rows a pass
  * takes (M picks the kernel: the GEMV for 1-2 rows, the MFMA kernel from 3, whose chunks are 256 k up to K = 3072
- * against the GEMV's up to 2048). For inspection of block-float and bf16 weights (an int4 weight runs the GEMV at any
- * M; dr_launch_plan gives any launch's own plan); results depend only on what this returns. */
+ * against the GEMV's up to 2048). For inspection of block-float and bf16 weights (dr_launch_plan
+ * gives any launch's own plan, an int4 weight's and that of more than 128 rows among them); results depend only on what this returns. */
 int dr_plan(int k, int m, int32_t* chunks, int32_t* kch, int32_t* rows_per_pass);
 
 /* What dr_matmul would launch for this launch, for inspection (replaces the plan dict that dense_reader/linear.py:
  * 455-495 choose/plan return): the kernel, the output tile width, the work split and the top-k records it writes. */
 typedef struct dr_launch_info {
-    int32_t kernel;        /* 0: the VALU GEMV (rows <= 2 a pass, and int4), 1: an MFMA kernel */
+    int32_t kernel;        /* 0: the VALU GEMV (rows <= 2, int4 <= 5), 1: an MFMA kernel */
     int32_t rows_per_pass; /* (from 129 rows on one launch takes all rows: its workgroups' rows, 64 to 256) */
     int32_t tile_cols;     /* output columns of a work tile: 16 (one panel) or 32 */
     int32_t tiles;         /* work tiles of the launch */

@@ -1820,6 +1820,90 @@ __device__ __forceinline__ void mgroup_bf16(const Args& a, const uint8_t* const*
             for (int tt = 0; tt < MT; ++tt) acc[q][tt] = mfma(A[u][tt], c[u][q], acc[q][tt]);
 }
 
+// int4 (W4A16), NB blocks of 128 k from b0. A lane's 16 bytes are its column's 32 k of one scale group (kq), and an MFMA
+// must sum one group's k over its four lane rows: the lane rows' dwords are transposed (dword D of lane row kq to register
+// kq of lane row D: four swaps a block), so that MFMA g takes k = 128 b + 32 g + 8 kq + j, all of group g. The weights
+// enter as the exact bf16 q, each group's products are summed from zero and the sum, scaled once by the lane's column's
+// scale, is added to the accumulator: one FMA a value of the accumulator and group, no x sum to take off again (the
+// GEMV's 136).
+__device__ __forceinline__ void swap_rows32(uint32_t& a, uint32_t& b) {  // a's lane rows 2, 3 with b's 0, 1
+    const auto v = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = v[0];
+    b = v[1];
+}
+__device__ __forceinline__ void swap_rows16(uint32_t& a, uint32_t& b) {  // a's lane rows 1, 3 with b's 0, 2
+    const auto v = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = v[0];
+    b = v[1];
+}
+// the 8 values q = u - 8 of a dword (k in nibble order: low nibbles k 0 .. 3, high 4 .. 7) as bf16
+__device__ __forceinline__ uint4 b_int4(uint32_t w) {
+    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+    float p[8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[j] = (float)((lo >> (8 * j)) & 0xFFu) - 8.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p[4 + j] = (float)((hi >> (8 * j)) & 0xFFu) - 8.f;
+    return make_uint4(pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7]));
+}
+template <int MT, int PW, int NB>
+__device__ __forceinline__ void mgroup_int4(const Args& a, const uint8_t* const* cb, const uint16_t* const* gs, int b0,
+                                            int lane, f32x4 (&acc)[PW][MT]) {
+    const int r = lane & 15, kq = lane >> 4;
+    uint4 A[NB][4][MT], c[NB][PW];
+    uint32_t sc[NB][PW];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int tt = 0; tt < MT; ++tt) A[b][g][tt] = x_row8(a, 16 * tt + r, (b0 + b) * 128 + 32 * g + 8 * kq);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < PW; ++q) sc[b][q] = __builtin_nontemporal_load(gs[q] + (size_t)(b0 + b) * 64 + lane);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < PW; ++q) c[b][q] = ld_stream16(cb[q] + (uint32_t)((b0 + b) * 1024 + lane * 16));
+    if (a.k != a.k_pad && (b0 + NB) * 128 > a.k) {  // (a ragged K's last blocks only)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int tt = 0; tt < MT; ++tt) x_kmask(A[b][g][tt], a, (b0 + b) * 128 + 32 * g + 8 * kq);
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < PW; ++q) {
+            uint32_t w[4] = {c[b][q].x, c[b][q].y, c[b][q].z, c[b][q].w};
+            swap_rows32(w[0], w[2]);
+            swap_rows32(w[1], w[3]);
+            swap_rows16(w[0], w[1]);
+            swap_rows16(w[2], w[3]);
+            // the column's scale of each group in every lane row
+            uint32_t s[4] = {sc[b][q], 0u, sc[b][q], 0u};
+            swap_rows32(s[0], s[2]);
+            s[1] = s[0];
+            s[3] = s[2];
+            swap_rows16(s[0], s[1]);
+            swap_rows16(s[2], s[3]);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const uint4 B = b_int4(w[g]);
+                const float sv = bf16_to_f32(s[g]);
+#pragma unroll
+                for (int tt = 0; tt < MT; ++tt) {
+                    const f32x4 t = mfma(A[b][g][tt], B, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[q][tt][j] = __builtin_fmaf(t[j], sv, acc[q][tt][j]);
+                }
+            }
+        }
+}
+
 // ---- 32 rows: a wavefront's chunk in steps of 128 k, software-pipelined ---------------------------------------------
 //
 // Step s + 1's x is staged and its codes loaded while step s is decoded and multiplied, so one step's loads are in
@@ -2137,10 +2221,23 @@ __global__ __launch_bounds__(512, MT == 2 ? 4 : 1) void dr_mfma(const Args a) { 
 #pragma unroll
         for (int tt = 0; tt < MT; ++tt) acc[q][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
     // 32 rows: x through the wavefront's LDS staging, which the partial sums overwrite after the K loop
-    constexpr bool XL = MT == 2;
+    constexpr bool XL = MT == 2 && FMT != DR_INT4;
     uint4* xs = reinterpret_cast<uint4*>(part) + wave * (XS_BYTES / 16);
     const int ch1 = min((split + 1) * a.cps, a.chunks);
-    if constexpr (XL) {
+    if constexpr (FMT == DR_INT4) {
+        const uint16_t* gs[PW];
+#pragma unroll
+        for (int q = 0; q < PW; ++q) gs[q] = sg.gscale + (size_t)(PW * t + q) * (a.k_pad / 128) * 64;
+        const int g0 = (split * a.cps * a.kch) >> 8, g1 = min(ch1 * a.kch, a.k_pad) >> 8;
+        for (int gg = g0 + wave; gg < g1; gg += a.waves) {
+            if constexpr (MT == 1) {
+                mgroup_int4<MT, PW, 2>(a, cb, gs, 2 * gg, lane, acc);
+            } else {
+                mgroup_int4<MT, PW, 1>(a, cb, gs, 2 * gg, lane, acc);
+                mgroup_int4<MT, PW, 1>(a, cb, gs, 2 * gg + 1, lane, acc);
+            }
+        }
+    } else if constexpr (XL) {
         for (int ch = split * a.cps + wave; ch < ch1; ch += a.waves) {
             const int k0 = ch * a.kch, k1 = min(k0 + a.kch, a.k_pad);
             if (fmt == DR_BFP8) xl_chunk_bfp8<PW>(a, cb, eb, k0, k1, lane, acc, xs);
@@ -2810,6 +2907,13 @@ int rows_per_pass(int m) {
     return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : 8;
 }
 
+// int4's rows a pass: the GEMV up to 5 rows (whose rows equal the one-token call's bit for bit), four a pass from 3 on,
+// then the MFMA kernel.
+#ifndef DR_INT4_MFMA_M
+#define DR_INT4_MFMA_M 6
+#endif
+int int4_rows(int m) { return m >= DR_INT4_MFMA_M ? (m <= 16 ? 16 : 32) : m <= 2 ? m : 4; }
+
 // Set by dr_launch_plan while it walks the launch path: the dense launches then store their kernel's LDS bytes (static
 // plus dynamic) here instead of launching it.
 thread_local size_t* lds_query = nullptr;
@@ -2877,13 +2981,15 @@ void launch_gemv(const Args& a, int grid, hipStream_t st) {
                 fire((dr_gemv<MR, PW, DR_BFP4, true>), dim3(grid), b, lds, st, a);
             break;
         case DR_INT4:
-            if constexpr (PW <= 2 && MR <= 2) {
-                if (plain) {
-                    if (g1)
-                        fire((dr_gemv_g1<MR, PW, DR_INT4, true, true>), dim3(grid), b, lds, st, a);
-                    else
-                        fire((dr_gemv<MR, PW, DR_INT4, true, true>), dim3(grid), b, lds, st, a);
-                    break;
+            if constexpr (PW <= 2 && MR <= 4) {
+                if constexpr (MR <= 2) {
+                    if (plain) {
+                        if (g1)
+                            fire((dr_gemv_g1<MR, PW, DR_INT4, true, true>), dim3(grid), b, lds, st, a);
+                        else
+                            fire((dr_gemv<MR, PW, DR_INT4, true, true>), dim3(grid), b, lds, st, a);
+                        break;
+                    }
                 }
                 if (g1)
                     fire((dr_gemv_g1<MR, PW, DR_INT4, true>), dim3(grid), b, lds, st, a);
@@ -2908,6 +3014,9 @@ void launch_mfma(const Args& a, int grid, hipStream_t st) {
     switch (a.seg[0].fmt) {
         case DR_BFP8: fire((dr_mfma<MT, PW, DR_BFP8, true>), dim3(grid), b, lds, st, a); break;
         case DR_BFP4: fire((dr_mfma<MT, PW, DR_BFP4, true>), dim3(grid), b, lds, st, a); break;
+        case DR_INT4:
+            if constexpr (PW <= 2) fire((dr_mfma<MT, PW, DR_INT4, true>), dim3(grid), b, lds, st, a);
+            break;
         default: fire((dr_mfma<MT, PW, DR_BF16, true>), dim3(grid), b, lds, st, a); break;
     }
 }
@@ -3197,7 +3306,16 @@ int prepare(const dr_launch* L, Args& a, int& pw, int& tiles, int& mr, bool gath
     mr = rows_per_pass(L->m);
     if (pw == 4 && mr == 8) mr = 4;    // (GLU: at most 4 GEMV rows or 16 MFMA rows a pass, for the registers
     if (pw == 4 && mr == 32) mr = 16;  // and the LDS)
-    if (a.seg[0].fmt == DR_INT4) mr = L->m >= 2 ? 2 : 1;  // (int4: the GEMV, two rows a pass)
+    if (a.seg[0].fmt == DR_INT4) {
+        // (fewer rows a pass where their split-K sums would not fit the library's own workspace)
+        mr = int4_rows(L->m);
+        const int narrower[] = {16, 4, 2};
+        for (const int r : narrower) {
+            plan(L->k, mr >= 16, &a.chunks, &a.kch, &a.waves, &a.splits, &a.cps);
+            if (a.splits == 1 || (int64_t)SPLIT_MAXTILES * 4 + (int64_t)tiles * a.splits * pw * mr * 16 * 4 <= DR_SCRATCH_BYTES) break;
+            if (r < mr) mr = r;
+        }
+    }
     plan(L->k, !gather && mr >= 16, &a.chunks, &a.kch, &a.waves, &a.splits, &a.cps);  // (the expert gather: as before)
     a.tiles = tiles;
     limit_splits(a);
@@ -3224,7 +3342,7 @@ int prepare(const dr_launch* L, Args& a, int& pw, int& tiles, int& mr, bool gath
     // 32 rows, plain tiles, more tiles than CUs: block-float segments in tile pairs (dr_mfma_pairs)
     a.pairs = 0;
     bool pairable = false;
-    for (int i = 0; i < a.nseg; ++i) pairable |= a.seg[i].fmt != DR_BF16;
+    for (int i = 0; i < a.nseg; ++i) pairable |= a.seg[i].fmt == DR_BFP8 || a.seg[i].fmt == DR_BFP4;
     if (!gather && pairable && mr == 32 && pw == 2 && a.splits == 1 && a.rec == nullptr && a.res == nullptr &&
         tiles > cu_count()) {
         // here a workgroup's bytes order the segments (a bfloat8_b pair 2 x 1088 B a 32-k step, a bf16 tile 2048, a
@@ -3341,7 +3459,8 @@ int run_passes(const dr_launch* L, const Args& a, int tiles, int mr, int pw, hip
         if (a.rec != nullptr && r0 >= a.tk_rows && !a.write_y) continue;
         // a last pass of at most 16 rows of a 32-row launch runs the 16-row MFMA kernel: the same plan, and each row's
         // sums the same bit for bit, at less cost (bfloat8_b K = 2048 N = 4096: 16 rows 7.4 us against 9.2 at 32)
-        const int rows = (mr == 32 && p.m <= 16) ? 16 : mr;
+        // (and int4's last GEMV pass the kernel of its rows: each row's sums are the same)
+        const int rows = (mr == 32 && p.m <= 16) ? 16 : (mr == 4 && a.seg[0].fmt == DR_INT4 && p.m <= 2) ? p.m : mr;
         hipError_t e = launch_rows(p, rows, pw, tiles * a.splits, st);
         if (e == hipSuccess && a.rec != nullptr && a.tk_group > 1 && r0 < a.tk_rows) {
             const int records = (tiles + a.tk_group - 1) / a.tk_group;

@@ -108,8 +108,8 @@ def w4a16_linear(x, wq, scale, *, memory_config=None, fidelity="hifi2", **opts):
 
 
 def rows_matmul(x2, wq, scale):
-    """y [M, N] bf16 = x2 [M, K] (bf16, GPU) @ (q * s).T: dr_matmul with a DR_INT4 segment, any M (the library runs
-    its GEMV two rows a pass)."""
+    """y [M, N] bf16 = x2 [M, K] (bf16, GPU) @ (q * s).T: dr_matmul with a DR_INT4 segment, any M (up to 5 rows on
+    the GEMV, each row's result that of a one-token call; more on the MFMA kernel, 16 or 32 a pass)."""
     L, y, x2 = _launch(x2, wq, scale)
     need = _lib.lib().dr_workspace_bytes(L)
     _lib.check(_lib.DR_EINVAL if need < 0 else _lib.DR_OK, "dr_workspace_bytes")
