@@ -2590,74 +2590,112 @@ __device__ __forceinline__ uint32_t bfp_face_row(const float (&v)[16], int (&sm)
 
 __device__ __forceinline__ uint32_t bf16_rne_bits(float f) { return f32_to_bf16(f); }
 
-template <int FMT>
+// A wavefront packs one panel over PACK_K values of k, 8 consecutive k of all 16 columns a lane. VEC (16-byte aligned
+// rows of w): a lane's loads are 32 of 16 bytes, all issued before any is used, columns past n read the last column's
+// (then zeroed); otherwise, and past K, value by value. The codes and exponents go out through LDS (16-byte slot c of
+// each run of 16 at c ^ (the run's index), which spreads the lanes' writes over the banks), so that the wavefront writes
+// whole 1 KiB blocks: written from the lanes directly they were 8-byte pieces and single exponent bytes, and with one
+// guarded load a value the pack of bfloat8_b K = 4096 N = 14336 took 130 us (80 now, 3.7 TB/s of the float values and the codes).
+constexpr int PACK_K = 512;
+
+template <int FMT, bool VEC>
 __global__ __launch_bounds__(256) void dr_pack_k(const float* __restrict__ w, long long ld_w, int n, int k,
                                                  const float* __restrict__ cdiv, uint8_t* __restrict__ codes,
                                                  uint8_t* __restrict__ exps, int n_pad, int k_pad) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int kgroups = k_pad / 8;
-    const long long total = (long long)(n_pad / 16) * kgroups;
-    if (idx >= total) return;
-    const int p = (int)(idx / kgroups), kg = (int)(idx % kgroups);
-    const int nkb = k_pad / kblk(FMT);
-    const int kk0 = kg * 8;
+    constexpr int WB = PACK_K * 16 * (FMT == DR_BFP8 ? 2 : FMT == DR_BFP4 ? 1 : 4) / 2;  // code bytes a wavefront
+    __shared__ uint4 lc[4][WB / 16];
+    __shared__ uint2 le[4][PACK_K / 8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int segs = (k_pad + PACK_K - 1) / PACK_K;
+    const long long item = (long long)blockIdx.x * 4 + wave;
+    if (item >= (long long)(n_pad / 16) * segs) return;  // (wavefronts work on their own: no barrier below)
+    const int p = (int)(item / segs), kb = (int)(item % segs) * PACK_K, kk0 = kb + 8 * lane;
     float v[8][16];
+    const bool whole = VEC && kk0 + 8 <= k;
+    if (whole) {
+        float4 t[16][2];
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
-        const int col = p * 16 + c;
-        const float d = (cdiv != nullptr && col < n) ? cdiv[col] : 1.f;
+        for (int c = 0; c < 16; ++c) {
+            const float* row = w + (long long)min(p * 16 + c, n - 1) * ld_w + kk0;
+            t[c][0] = *reinterpret_cast<const float4*>(row);
+            t[c][1] = *reinterpret_cast<const float4*>(row + 4);
+        }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int kk = kk0 + i;
-            float x = (col < n && kk < k) ? w[(long long)col * ld_w + kk] : 0.f;
-            if (cdiv != nullptr && col < n) x = x / d;
-            v[i][c] = x;
+        for (int c = 0; c < 16; ++c) {
+            const bool in = p * 16 + c < n;
+            const float x[8] = {t[c][0].x, t[c][0].y, t[c][0].z, t[c][0].w, t[c][1].x, t[c][1].y, t[c][1].z, t[c][1].w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i][c] = in ? x[i] : 0.f;
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int col = p * 16 + c, kk = kk0 + i;
+                v[i][c] = (col < n && kk < k) ? w[(long long)col * ld_w + kk] : 0.f;
+            }
+    }
+    if (cdiv != nullptr) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const int col = p * 16 + c;
+            if (col < n) {
+                const float d = cdiv[col];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i][c] = v[i][c] / d;
+            }
         }
     }
-    uint8_t* pbase = codes + (size_t)p * nkb * 1024;
+    // run: the 16 slots (16 columns) of one k-block's quarter that the lane writes into
+    const int run = FMT == DR_BFP8 ? lane >> 1 : FMT == DR_BFP4 ? lane >> 2 : lane;
+    uint8_t* lb = reinterpret_cast<uint8_t*>(lc[wave]);
+    auto slot = [&](int c) { return lb + (run * 16 + (c ^ (run & 15))) * 16; };
     if (FMT == DR_BF16) {
-        const int b = kk0 / 32, kq = (kk0 % 32) / 8;
 #pragma unroll
         for (int c = 0; c < 16; ++c) {
             uint32_t h[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) h[i] = bf16_rne_bits(v[i][c]);
-            const uint4 o = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
-            *reinterpret_cast<uint4*>(pbase + (size_t)b * 1024 + (kq * 16 + c) * 16) = o;
-        }
-        return;
-    }
-    int sm[8][16];
-    uint32_t ex[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ex[i] = bfp_face_row<FMT == DR_BFP8 ? 7 : 3>(v[i], sm[i]);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) exps[(size_t)p * k_pad + exp_off(FMT, kk0 + i)] = (uint8_t)ex[i];
-    if (FMT == DR_BFP8) {
-        const int b = kk0 / 64, kq = (kk0 % 64) / 16, off = kk0 % 16;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            uint32_t lo = 0, hi = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                lo |= ((uint32_t)sm[i][c] & 0xFFu) << (8 * i);
-                hi |= ((uint32_t)sm[4 + i][c] & 0xFFu) << (8 * i);
-            }
-            *reinterpret_cast<uint2*>(pbase + (size_t)b * 1024 + (kq * 16 + c) * 16 + off) = make_uint2(lo, hi);
+            *reinterpret_cast<uint4*>(slot(c)) =
+                make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
         }
     } else {
-        const int b = kk0 / 128, kq = (kk0 % 128) / 32, d = (kk0 % 32) / 8;
+        int sm[8][16];
+        uint8_t* leb = reinterpret_cast<uint8_t*>(le[wave]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) leb[exp_off(FMT, 8 * lane + i)] = (uint8_t)bfp_face_row<FMT == DR_BFP8 ? 7 : 3>(v[i], sm[i]);
 #pragma unroll
         for (int c = 0; c < 16; ++c) {
-            uint32_t word = 0;
+            if (FMT == DR_BFP8) {
+                uint32_t lo = 0, hi = 0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t ulo = (uint32_t)(sm[j][c] + 8), uhi = (uint32_t)(sm[4 + j][c] + 8);
-                word |= (ulo | (uhi << 4)) << (8 * j);
+                for (int i = 0; i < 4; ++i) {
+                    lo |= ((uint32_t)sm[i][c] & 0xFFu) << (8 * i);
+                    hi |= ((uint32_t)sm[4 + i][c] & 0xFFu) << (8 * i);
+                }
+                *reinterpret_cast<uint2*>(slot(c) + 8 * (lane & 1)) = make_uint2(lo, hi);
+            } else {
+                uint32_t word = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t ulo = (uint32_t)(sm[j][c] + 8), uhi = (uint32_t)(sm[4 + j][c] + 8);
+                    word |= (ulo | (uhi << 4)) << (8 * j);
+                }
+                *reinterpret_cast<uint32_t*>(slot(c) + 4 * (lane & 3)) = word;
             }
-            *reinterpret_cast<uint32_t*>(pbase + (size_t)b * 1024 + (kq * 16 + c) * 16 + d * 4) = word;
         }
     }
+    // (the wavefront's own LDS, written before it is read: its LDS instructions run in order)
+    __builtin_amdgcn_wave_barrier();
+    const int part = min(k_pad - kb, PACK_K);  // (256 of them in the last segment of an odd number of groups)
+    uint8_t* out = codes + (size_t)p * (k_pad / kblk(FMT)) * 1024 + (size_t)(kb / kblk(FMT)) * 1024;
+#pragma unroll
+    for (int i = 0; i < WB / 1024; ++i) {
+        const int sl = 64 * i + lane, g = sl >> 4;
+        if (1024 * i < WB / PACK_K * part) reinterpret_cast<uint4*>(out)[sl] = lc[wave][g * 16 + ((sl & 15) ^ (g & 15))];
+    }
+    if (FMT != DR_BF16 && 8 * lane < part) reinterpret_cast<uint2*>(exps + (size_t)p * k_pad + kb)[lane] = le[wave][lane];
 }
 
 // DR_BFP4_KB: one thread a (column, 16-k group): the group's shared exponent and its 16 codes (bfloat4_b's rounding,
@@ -2695,35 +2733,68 @@ __global__ __launch_bounds__(256) void dr_pack_kb_k(const float* __restrict__ w,
         make_uint2(word[0], word[1]);
 }
 
+// the values of a lane's 16 bytes (block b of its 256-k group) in k order
+template <int FMT, int I = 0, typename F>
+__device__ __forceinline__ void unpack_row(const uint32_t (&w)[4], uint32_t e, int b, F put) {
+    constexpr int PER = kblk(FMT) / 4;
+    if constexpr (I < PER) {
+        float v;
+        if constexpr (FMT == DR_BF16) {
+            v = bf16_to_f32((w[I / 2] >> (16 * (I % 2))) & 0xFFFFu);
+        } else if constexpr (FMT == DR_BFP8) {
+            const int m = (int)(signed char)(w[I / 4] >> (8 * (I % 4)));
+            const uint32_t ew = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e, 0x150 + I, 0xF, 0xF, true);
+            v = __builtin_ldexpf((float)m, (int)((ew >> (8 * b)) & 0xFFu) - 133);
+        } else {
+            const int m = (int)((w[I / 8] >> (8 * (I % 4) + (I % 8 < 4 ? 0 : 4))) & 15u) - 8;
+            uint32_t ev;
+            if constexpr (FMT == DR_BFP4_KB) {
+                ev = e >> (8 * (I / 16));
+            } else {
+                const uint32_t ew = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e, 0x150 + I / 2, 0xF, 0xF, true);
+                ev = ew >> (16 * b + 8 * (I % 2));
+            }
+            v = __builtin_ldexpf((float)m, (int)(ev & 0xFFu) - 129);
+        }
+        put(I, v);
+        unpack_row<FMT, I + 1>(w, e, b, put);
+    }
+}
+
+// A wavefront writes 64 columns (four panels, a column a lane) over 256 k of out: a lane's 16-byte loads hold
+// consecutive k of its column, each value's row of 64 columns is one 256-byte store, and the panel's exponents, a dword
+// a lane, are broadcast across the 16 lanes of the panel. (One thread a value, with its 64-bit divisions and byte loads,
+// took 152 us for bfloat8_b K = 4096 N = 14336; 75 us now, 4.0 TB/s.)
 template <int FMT>
 __global__ __launch_bounds__(256) void dr_unpack_k(const uint8_t* __restrict__ codes, const uint8_t* __restrict__ exps,
-                                                   int n, int k, int k_pad, float* __restrict__ out, long long ld_out) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)n * k) return;
-    const int kk = (int)(idx / n), col = (int)(idx % n);
-    const int p = col / 16, c = col % 16;
-    const int nkb = k_pad / kblk(FMT);
-    const uint8_t* pbase = codes + (size_t)p * nkb * 1024;
-    float val;
-    if (FMT == DR_BF16) {
-        const int b = kk / 32, kq = (kk % 32) / 8, i = kk % 8;
-        const uint16_t h = *reinterpret_cast<const uint16_t*>(pbase + (size_t)b * 1024 + (kq * 16 + c) * 16 + 2 * i);
-        val = bf16_to_f32(h);
-    } else {
-        const int e = exps[(size_t)p * k_pad + (FMT == DR_BFP4_KB ? exp_off_kb(kk, c) : exp_off(FMT, kk))];
-        int m;
-        if (FMT == DR_BFP8) {
-            const int b = kk / 64, kq = (kk % 64) / 16, i = kk % 16;
-            m = (int)(signed char)pbase[(size_t)b * 1024 + (kq * 16 + c) * 16 + i];
-            val = __builtin_ldexpf((float)m, e - 133);
-        } else {
-            const int b = kk / 128, kq = (kk % 128) / 32, d = (kk % 32) / 8, j = kk % 8;
-            const uint8_t byte = pbase[(size_t)b * 1024 + (kq * 16 + c) * 16 + d * 4 + (j & 3)];
-            m = (int)((j < 4 ? byte : (byte >> 4)) & 15) - 8;
-            val = __builtin_ldexpf((float)m, e - 129);
+                                                   int n, int k, int n_pad, int k_pad, float* __restrict__ out,
+                                                   long long ld_out) {
+    constexpr int KB = kblk(FMT), PER = KB / 4;  // k of a block, of a lane's load
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15;
+    const int groups = (k + 255) / 256;
+    const long long item = (long long)blockIdx.x * 4 + wave;
+    if (item >= (long long)((n + 63) / 64) * groups) return;
+    const int n0 = (int)(item / groups) * 64, g = (int)(item % groups);
+    const int p = min((n0 + lane) >> 4, n_pad / 16 - 1), col = n0 + lane;
+    const uint8_t* pc = codes + (size_t)p * (k_pad / KB) * 1024 + (size_t)(g * (256 / KB)) * 1024 + c * 16;
+    const uint8_t* pe = FMT == DR_BF16 ? nullptr : exps + (size_t)p * k_pad + g * 256;
+    for (int kq = 0; kq < 4; ++kq) {
+        // bfp8 / bfp4: this lane's exponents (its k of each block, or its pair of k); kblock: the lane's column's own
+        uint32_t e = 0;
+        if (FMT == DR_BFP8 || FMT == DR_BFP4) e = *reinterpret_cast<const uint32_t*>(pe + 4 * (16 * kq + c));
+#pragma unroll
+        for (int b = 0; b < 256 / KB; ++b) {
+            const uint4 q = *reinterpret_cast<const uint4*>(pc + b * 1024 + kq * 256);
+            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+            if (FMT == DR_BFP4_KB) e = *reinterpret_cast<const uint16_t*>(pe + b * 128 + (kq * 16 + c) * 2);
+            const int kk = g * 256 + b * KB + kq * PER;
+            float* o = out + (long long)kk * ld_out + col;
+            auto put = [&](int i, float v) {
+                if (kk + i < k && col < n) o[(long long)i * ld_out] = v;
+            };
+            unpack_row<FMT>(w, e, b, put);
         }
     }
-    out[(long long)kk * ld_out + col] = val;
 }
 
 // int4 codes q [n][ldq] (-7..7) to the bfloat4_b code layout (u = q + 8): one thread per (panel, k-block, lane), the
@@ -3158,8 +3229,9 @@ int dr_pack(const float* w, int64_t ld_w, int n, int k, int fmt, const float* co
         k_pad % KALIGN || ld_w < k || (fmt != DR_BF16 && exps == nullptr) || fmt < 0 || fmt > DR_BFP4_KB ||
         fmt == DR_INT4)
         return DR_EINVAL;
-    const long long total = (long long)(n_pad / 16) * (k_pad / 8);
-    const int grid = (int)((total + 255) / 256);
+    const long long items = (long long)(n_pad / 16) * ((k_pad + PACK_K - 1) / PACK_K);
+    const dim3 grid((unsigned)((items + 3) / 4)), blk(256);
+    const bool vec = ld_w % 4 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
     auto* c8 = reinterpret_cast<uint8_t*>(codes);
     auto* e8 = reinterpret_cast<uint8_t*>(exps);
     if (fmt == DR_BFP4_KB) {
@@ -3167,11 +3239,11 @@ int dr_pack(const float* w, int64_t ld_w, int n, int k, int fmt, const float* co
         hipLaunchKernelGGL(dr_pack_kb_k, dim3((int)((tk + 255) / 256)), dim3(256), 0, S(stream), w, (long long)ld_w, n, k,
                            col_div, c8, e8, n_pad, k_pad);
     } else if (fmt == DR_BFP8)
-        hipLaunchKernelGGL(dr_pack_k<DR_BFP8>, dim3(grid), dim3(256), 0, S(stream), w, (long long)ld_w, n, k, col_div, c8, e8, n_pad, k_pad);
+        hipLaunchKernelGGL((vec ? dr_pack_k<DR_BFP8, true> : dr_pack_k<DR_BFP8, false>), grid, blk, 0, S(stream), w, (long long)ld_w, n, k, col_div, c8, e8, n_pad, k_pad);
     else if (fmt == DR_BFP4)
-        hipLaunchKernelGGL(dr_pack_k<DR_BFP4>, dim3(grid), dim3(256), 0, S(stream), w, (long long)ld_w, n, k, col_div, c8, e8, n_pad, k_pad);
+        hipLaunchKernelGGL((vec ? dr_pack_k<DR_BFP4, true> : dr_pack_k<DR_BFP4, false>), grid, blk, 0, S(stream), w, (long long)ld_w, n, k, col_div, c8, e8, n_pad, k_pad);
     else
-        hipLaunchKernelGGL(dr_pack_k<DR_BF16>, dim3(grid), dim3(256), 0, S(stream), w, (long long)ld_w, n, k, col_div, c8, e8, n_pad, k_pad);
+        hipLaunchKernelGGL((vec ? dr_pack_k<DR_BF16, true> : dr_pack_k<DR_BF16, false>), grid, blk, 0, S(stream), w, (long long)ld_w, n, k, col_div, c8, e8, n_pad, k_pad);
     return hip_status(hipGetLastError());
 }
 
@@ -3180,18 +3252,18 @@ int dr_unpack(const void* codes, const void* exps, int fmt, int n, int k, int n_
     if (codes == nullptr || out == nullptr || n <= 0 || k <= 0 || n > n_pad || k > k_pad || k_pad % KALIGN ||
         n_pad % 32 || ld_out < n || (fmt != DR_BF16 && exps == nullptr) || fmt < 0 || fmt > DR_BFP4_KB || fmt == DR_INT4)
         return DR_EINVAL;
-    const long long total = (long long)n * k;
-    const int grid = (int)((total + 255) / 256);
+    const long long items = (long long)((n + 63) / 64) * ((k + 255) / 256);
+    const unsigned grid = (unsigned)((items + 3) / 4);
     auto* c8 = reinterpret_cast<const uint8_t*>(codes);
     auto* e8 = reinterpret_cast<const uint8_t*>(exps);
     if (fmt == DR_BFP8)
-        hipLaunchKernelGGL(dr_unpack_k<DR_BFP8>, dim3(grid), dim3(256), 0, S(stream), c8, e8, n, k, k_pad, out, (long long)ld_out);
+        hipLaunchKernelGGL(dr_unpack_k<DR_BFP8>, dim3(grid), dim3(256), 0, S(stream), c8, e8, n, k, n_pad, k_pad, out, (long long)ld_out);
     else if (fmt == DR_BFP4)
-        hipLaunchKernelGGL(dr_unpack_k<DR_BFP4>, dim3(grid), dim3(256), 0, S(stream), c8, e8, n, k, k_pad, out, (long long)ld_out);
+        hipLaunchKernelGGL(dr_unpack_k<DR_BFP4>, dim3(grid), dim3(256), 0, S(stream), c8, e8, n, k, n_pad, k_pad, out, (long long)ld_out);
     else if (fmt == DR_BFP4_KB)
-        hipLaunchKernelGGL(dr_unpack_k<DR_BFP4_KB>, dim3(grid), dim3(256), 0, S(stream), c8, e8, n, k, k_pad, out, (long long)ld_out);
+        hipLaunchKernelGGL(dr_unpack_k<DR_BFP4_KB>, dim3(grid), dim3(256), 0, S(stream), c8, e8, n, k, n_pad, k_pad, out, (long long)ld_out);
     else
-        hipLaunchKernelGGL(dr_unpack_k<DR_BF16>, dim3(grid), dim3(256), 0, S(stream), c8, e8, n, k, k_pad, out, (long long)ld_out);
+        hipLaunchKernelGGL(dr_unpack_k<DR_BF16>, dim3(grid), dim3(256), 0, S(stream), c8, e8, n, k, n_pad, k_pad, out, (long long)ld_out);
     return hip_status(hipGetLastError());
 }
 
@@ -3396,7 +3468,10 @@ void bind_split(Args& a, void* workspace, int pw, int mr) {
 // K = 4096 N = 14336 70, 114, 449 -> 50, 51, 113 us; K = 14336 N = 4096 104, 165, 648 -> 60, 63, 172; K = 1024 N = 1024
 // 37, 44, 180 -> 14 (the call's host time). Up to 128 rows the passes stay: their rows equal those of a call on them
 // alone bit for bit.
-constexpr int GEMM_MIN_M = 129;
+// A GLU's passes are 16 rows, and it goes over from 33 rows on (a block list's single calls, up to 32 rows, keep the
+// passes' sums): bfloat8_b gate
+// and up K = 4096 N = 14336 at 33, 64 and 128 rows 78, 107, 215 -> 45, 45, 51 us, bfloat4_b 58, 78, 157 -> 41, 42, 50.
+constexpr int GEMM_MIN_M = 129, GEMM_MIN_M_GLU = 33;
 
 // The tile: mt row tiles of 32 with the wavefronts side by side (256 columns a workgroup, 128 with a GLU), or ks, 64
 // rows x 64 columns with the wavefronts splitting K. The one of the least time by rounds of workgroups over the CUs
@@ -3412,7 +3487,7 @@ constexpr GemmTile GEMM_TILES[] = {{2, true, 100, 28}, {2, false, 300, 66}, {4, 
 
 // false: the launch runs in passes
 bool gemm_plan(const dr_launch* L, const Args& a, GemmArgs& g, GemmTile& best) {
-    if (L->m < GEMM_MIN_M || a.nseg != 1 || a.rec != nullptr || a.seg[0].fmt > DR_BF16) return false;
+    if (L->m < (a.seg[0].glu ? GEMM_MIN_M_GLU : GEMM_MIN_M) || a.nseg != 1 || a.rec != nullptr || a.seg[0].fmt > DR_BF16) return false;
     const SegDev& s = a.seg[0];
     g = GemmArgs{};
     g.x = a.x;

@@ -98,7 +98,7 @@ def test_epilogue(device, fmt, m, k, n):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", list(FMTS))
-@pytest.mark.parametrize("m, k, n", [(129, 800, 96), (150, 256, 7200), (333, 288, 8224), (600, 96, 8192)])
+@pytest.mark.parametrize("m, k, n", [(33, 96, 64), (65, 1056, 7200), (129, 800, 96), (150, 256, 7200), (333, 288, 8224), (600, 96, 8192)])
 def test_glu(device, fmt, m, k, n):
     """Gate and up apart (with column scales) and interleaved, silu and gelu_tanh."""
     gw, uw = O.matrix(n, k, 21), O.matrix(n, k, 22)
