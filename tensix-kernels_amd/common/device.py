@@ -88,6 +88,12 @@ class Device:
         return f"Device({self.id})"
 
 
+def raw_stream(device):
+    """The current HIP stream (its handle) of a torch GPU device, without the Stream object torch.cuda.current_stream
+    makes a call."""
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
+
+
 def open_device(device_id=0):
     return Device(device_id)
 

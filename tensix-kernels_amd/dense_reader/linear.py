@@ -193,7 +193,8 @@ def native_weight(device, t, dtype, col_scale=False, sharded=True, max_banks=Non
     rounding and multiplied back after the matmul (reference linear.py:144-156). The packing runs on the GPU."""
     d = dev.as_device(device)
     t = t.float()
-    c = bf16_ceil(t.abs().amax(dim=1).clamp(min=1e-8)) if col_scale else torch.ones(t.shape[0])
+    # (unit scales are made where they are used: a copy from the host would wait for the device)
+    c = bf16_ceil(t.abs().amax(dim=1).clamp(min=1e-8)) if col_scale else torch.ones(t.shape[0], device=d.torch)
     n, k = t.shape
     mc = sharded_memcfg(d, k, n, max_banks=max_banks) if sharded else MemoryConfig(0)
     n_pad = mc.banks * mc.shard_width if sharded else -(-n // TILE) * TILE
@@ -431,10 +432,12 @@ def choose_blocks(device, x, w, full_sync=False, **forced):
 
 
 def _x2d(x):
-    """x [..., M, K] with leading dims of 1 (or any rank <= 4 that flattens to rows) as a contiguous [M, K] bf16 whose
-    rows start 16-byte aligned (a copy when x's do not)."""
+    """x [..., M, K] with leading dims of 1 (or any rank <= 4 that flattens to rows) as contiguous bf16 rows of K that
+    start 16-byte aligned (x itself, or a copy [M, K] when its rows do not)."""
     assert isinstance(x, torch.Tensor) and x.is_cuda, "dense_reader: x is a bf16 torch tensor on the GPU"
     assert x.dtype == torch.bfloat16, (x.dtype, "dense_reader: x is bf16")
+    if x.is_contiguous() and x.data_ptr() % 16 == 0 and x.dim() > 0:
+        return x  # (its memory as it is: no view is needed)
     x2 = x.reshape(-1, x.shape[-1])
     if not x2.is_contiguous() or x2.data_ptr() % 16:  # (the kernels read x rows 16 bytes at a time)
         x2 = x2.contiguous() if not x2.is_contiguous() else x2.clone()
@@ -461,13 +464,14 @@ def _segment(seg, w, up, col0_tiles, scale, glu, scale_up=None):
     if up is not None:
         seg.codes_up = up.codes.data_ptr()
         seg.exps_up = up.exps_ptr()
-    p, f32 = _scale_ptr(scale, w.n)
-    seg.scale = p
-    pu, f32u = _scale_ptr(scale_up, w.n)
-    seg.scale_up = pu
-    if p is not None and pu is not None:
-        assert f32 == f32u, "dense_reader: gate and up scales of one dtype"
-    seg.scale_f32 = f32 or f32u
+    if scale is not None or scale_up is not None:
+        p, f32 = _scale_ptr(scale, w.n)
+        seg.scale = p
+        pu, f32u = _scale_ptr(scale_up, w.n)
+        seg.scale_up = pu
+        if p is not None and pu is not None:
+            assert f32 == f32u, "dense_reader: gate and up scales of one dtype"
+        seg.scale_f32 = f32 or f32u
     seg.col0 = TILE * col0_tiles
 
 
@@ -510,17 +514,30 @@ def matmul(
     one launch, one output, over two to four column blocks of one K; each block's columns go to its col0_tiles. The
     output equals one call per block (out=, col0=) bit for bit. Block output spans must not overlap."""
     L, y, keep = _launch(x, w, scale, topk=topk, out=out, col0=col0, w_up=w_up, max_banks=max_banks, **opts)
-    d = x.device
-    st = torch.cuda.current_stream(d)
-    L.stream = st.cuda_stream
-    need = _lib.lib().dr_workspace_bytes(L)
-    _lib.check(_lib.DR_EINVAL if need < 0 else _lib.DR_OK, "dr_workspace_bytes")
-    if need > 0:
-        ws = _workspace(d, st, need)
-        L.workspace, L.workspace_bytes = ws.data_ptr(), ws.numel()
-    _lib.check(_lib.lib().dr_matmul(L), "dr_matmul")
+    run(L, x.device, "dr_matmul")
     del keep
     return y
+
+
+def run(L, device, what):
+    """Enqueue a filled dr_launch on the device's current stream, with the stream's workspace if it has one: a launch
+    that needs more is refused before anything is enqueued, and only then its need is asked for and the workspace
+    grown (so a call costs one entry into the library, not two)."""
+    stream = dev.raw_stream(device)
+    L.stream = stream
+    ws = _WORKSPACE.get((device, stream, "matmul"))
+    if ws is not None:
+        L.workspace, L.workspace_bytes = ws.data_ptr(), ws.numel()
+    lib = _lib.lib()
+    st = lib.dr_matmul(L)
+    if st == _lib.DR_EINVAL:
+        need = lib.dr_workspace_bytes(L)
+        if need > 0 and need > L.workspace_bytes:
+            ws = _workspace(device, stream, need)
+            L.workspace, L.workspace_bytes = ws.data_ptr(), ws.numel()
+            st = lib.dr_matmul(L)
+    if st != _lib.DR_OK:
+        _lib.check(st, what)
 
 
 def launch_plan(x, w, scale, **kw):
@@ -568,13 +585,14 @@ def _launch(x, w, scale, *, topk=None, out=None, col0=0, w_up=None, max_banks=No
     assert not (out32 and topk is not None), "dense_reader: out32 without top-k"
     assert not (out32 and out is not None and out.dtype != torch.float32), out.dtype
     x2 = _x2d(x)
-    M, K = x2.shape
+    K = x.shape[-1]
+    M = x.numel() // K if K else 0
     glu = bool(opts.get("glu", False))
     act = opts.pop("glu_act", 0)  # the GLU's activation: 0 silu, 1 gelu_tanh
     assert act in (0, 1) and (act == 0 or glu), "dense_reader: glu_act (0 silu, 1 gelu_tanh) needs glu"
     first = entries[0][0] if entries else w
     assert native_tile(first), f"dense_reader: weights are bfloat8_b, bfloat4_b or bfloat16, not {getattr(first, 'dtype', first)}"
-    assert first.shape[-2] == K, (x.shape, first.shape)
+    assert first.k == K, (x.shape, first.shape)
     if w_up is not None:
         assert glu, "dense_reader: w_up is the GLU's up weight (glu=True)"
         assert w_up.dtype == w.dtype and tuple(w_up.padded_shape) == tuple(w.padded_shape)
@@ -593,19 +611,20 @@ def _launch(x, w, scale, *, topk=None, out=None, col0=0, w_up=None, max_banks=No
         assert r2.shape[0] >= M and r2.shape[1] >= n_out, (residual.shape, M, n_out)
         assert r2.is_contiguous()
         assert col0 == 0 and (out is None or out is residual), "dense_reader: residual with a fresh output or in place"
-    y = out
-    if y is None:
-        y = torch.empty(1, 1, M, n_out, dtype=torch.float32 if out32 else torch.bfloat16, device=d)
+    y, ycols = out, n_out
     assert entries or col0 == 0 or (out is not None and topk is None), "dense_reader: col0 needs out, no top-k"
-    y2 = y.reshape(-1, y.shape[-1])
-    assert y2.shape[0] >= M and y.is_contiguous(), (y.shape, M)
-    assert y.dtype == (torch.float32 if out32 else torch.bfloat16), (y.dtype, out32)
+    if y is None:
+        y = torch.empty((1, 1, M, n_out), dtype=torch.float32 if out32 else torch.bfloat16, device=d)
+    else:
+        ycols = y.shape[-1]
+        assert y.numel() // max(ycols, 1) >= M and y.is_contiguous(), (y.shape, M)
+        assert y.dtype == (torch.float32 if out32 else torch.bfloat16), (y.dtype, out32)
     blocks = entries or [(w, w_up, col0, scale)]
     ends = []
     for g, u, c0, _ in blocks:
         nb = g.n // 2 if (glu and u is None) else g.n
         ends.append((c0, -(-nb // TILE)))
-        assert TILE * c0 + nb <= y2.shape[1], (c0, nb, y.shape)
+        assert TILE * c0 + nb <= ycols, (c0, nb, y.shape)
     if entries:
         spans = sorted(ends)
         assert all(a0 + an <= b0 for (a0, an), (b0, _) in itertools.pairwise(spans)), (
@@ -614,8 +633,8 @@ def _launch(x, w, scale, *, topk=None, out=None, col0=0, w_up=None, max_banks=No
     L = _lib.Launch()
     L.x = x2.data_ptr()
     L.m, L.k, L.ldx = M, K, K
-    L.y = y2.data_ptr()
-    L.ldy = y2.shape[1]
+    L.y = y.data_ptr()
+    L.ldy = ycols
     L.y_f32 = int(out32)
     if residual is not None:
         L.residual = r2.data_ptr()
@@ -623,8 +642,9 @@ def _launch(x, w, scale, *, topk=None, out=None, col0=0, w_up=None, max_banks=No
         L.residual_mode = res_mode
     L.act = act
     L.nseg = len(blocks)
+    segs = L.seg
     for i, (g, u, c0, sc) in enumerate(blocks):
-        _segment(L.seg[i], g, u, c0, sc, glu, scale_up if i == 0 else None)
+        _segment(segs[i], g, u, c0, sc, glu, scale_up if i == 0 else None)
     if topk is not None:
         assert M <= 32, "dense_reader: top-k needs one row slice (up to 32 rows)"
         r = topk["r"]
@@ -656,10 +676,10 @@ _WORKSPACE = {}
 
 def _workspace(device, stream, nbytes, kind="matmul"):
     """The workspace of one kind of launch (the matmul's split K, or the top-k merge and head pick) on a device and
-    stream: zeroed once when allocated (or grown); every launch leaves its counters at zero, each kind's counters lie
+    stream (dev.raw_stream's): zeroed once when allocated (or grown); every launch leaves its counters at zero, each kind's counters lie
     at one place whatever the launch's shape, and launches on one stream never overlap. The two kinds keep apart: each
     lays its counters out its own way."""
-    key = (device, stream.cuda_stream, kind)
+    key = (device, stream, kind)
     ws = _WORKSPACE.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
@@ -785,7 +805,7 @@ def topk_merge(r, rows, k, k_out=32, fp32=False, records=None):
     n = words.shape[0] if records is None else records
     vals = torch.empty(rows, k_out, dtype=torch.float32, device=r.device)
     ids = torch.empty(rows, k_out, dtype=torch.int32, device=r.device)
-    st = torch.cuda.current_stream(r.device)
+    st = dev.raw_stream(r.device)
     need = _lib.lib().dr_topk_merge_workspace_bytes(n, rows, k)
     _lib.check(_lib.DR_EINVAL if need < 0 else _lib.DR_OK, "dr_topk_merge_workspace_bytes")
     wp, wn = None, 0
@@ -793,7 +813,7 @@ def topk_merge(r, rows, k, k_out=32, fp32=False, records=None):
         ws = _workspace(r.device, st, need, "merge")
         wp, wn = ws.data_ptr(), ws.numel()
     st = _lib.lib().dr_topk_merge(
-        words.data_ptr(), n, rows, k, int(fp32), k_out, vals.data_ptr(), ids.data_ptr(), wp, wn, st.cuda_stream
+        words.data_ptr(), n, rows, k, int(fp32), k_out, vals.data_ptr(), ids.data_ptr(), wp, wn, st
     )
     _lib.check(st, "dr_topk_merge")
     return vals, ids

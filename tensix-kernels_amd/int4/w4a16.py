@@ -111,12 +111,7 @@ def rows_matmul(x2, wq, scale):
     """y [M, N] bf16 = x2 [M, K] (bf16, GPU) @ (q * s).T: dr_matmul with a DR_INT4 segment, any M (up to 5 rows on
     the GEMV, each row's result that of a one-token call; more on the MFMA kernel, 16 or 32 a pass)."""
     L, y, x2 = _launch(x2, wq, scale)
-    need = _lib.lib().dr_workspace_bytes(L)
-    _lib.check(_lib.DR_EINVAL if need < 0 else _lib.DR_OK, "dr_workspace_bytes")
-    if need > 0:
-        ws = linear._workspace(x2.device, torch.cuda.current_stream(x2.device), need)
-        L.workspace, L.workspace_bytes = ws.data_ptr(), ws.numel()
-    _lib.check(_lib.lib().dr_matmul(L), "dr_matmul (int4)")
+    linear.run(L, x2.device, "dr_matmul (int4)")
     return y
 
 
@@ -149,7 +144,6 @@ def _launch(x2, wq, scale):
     s0.fmt, s0.n, s0.n_pad = DR_INT4, n, wq["n_pad"]
     s0.codes, s0.exps = wq["t"].data_ptr(), None
     s0.scale = scale.data_ptr()
-    L.stream = torch.cuda.current_stream(x2.device).cuda_stream
     return L, y, x2
 
 

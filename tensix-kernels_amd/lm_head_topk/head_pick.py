@@ -106,12 +106,12 @@ def pick(records, x, rows_t, nrows, k, top=16, logits="bf16", out=None, valid=No
     assert out.dtype == torch.int32 and out.numel() >= TILE * TILE and out.is_contiguous(), (out.shape, out.dtype)
     if ids_out is not None:
         check_ids_out(ids_out)
-    stream = torch.cuda.current_stream(x.device)
+    stream = dev.raw_stream(x.device)
     wp, wn = _select_workspace(x.device, stream, words.shape[0], nrows, k)
     st = _lib.lib().dr_head_pick(
         words.data_ptr(), words.shape[0], nrows, k, top, int(logits == "bf16"), x2.data_ptr(), x2.shape[1], dim,
         rows_t.data_ptr(), dim, vocab, out.data_ptr(), None if ids_out is None else ids_out.data_ptr(), wp, wn,
-        stream.cuda_stream,
+        stream,
     )
     _lib.check(st, "dr_head_pick")
     return out
@@ -149,11 +149,11 @@ def pick_records(records, nrows, k, vocab, tmap=None, out=None, ids_out=None):
         out = _out_page(records.device)
     if ids_out is not None:
         check_ids_out(ids_out)
-    stream = torch.cuda.current_stream(records.device)
+    stream = dev.raw_stream(records.device)
     wp, wn = _select_workspace(records.device, stream, words.shape[0], nrows, k)
     st = _lib.lib().dr_head_pick_records(
         words.data_ptr(), words.shape[0], nrows, k, vocab, None if tmap is None else tmap.data_ptr(), out.data_ptr(),
-        None if ids_out is None else ids_out.data_ptr(), wp, wn, stream.cuda_stream,
+        None if ids_out is None else ids_out.data_ptr(), wp, wn, stream,
     )
     _lib.check(st, "dr_head_pick_records")
     return out

@@ -521,29 +521,39 @@ def _run(P, x2, m, k_launch, ldx, y, ldy, gate_up_mode, mode, ids, ids32, w, slo
     M.slots, M.id_rows, M.experts = slots, id_rows, P["E"]
     if gate_up_mode:
         s0.glu, s0.n, s0.n_pad = 2, P["I"], gn
-        s0.codes, s0.exps = P["gu"][0, 0].data_ptr(), P["gu_exps"][0, 0].data_ptr()
-        s0.codes_up, s0.exps_up = P["gu"][0, 1].data_ptr(), P["gu_exps"][0, 1].data_ptr()
+        # (expert 0's gate, then its up: [E, 2, codes] and [E, 2, exps])
+        s0.codes, s0.exps = P["gu"].data_ptr(), P["gu_exps"].data_ptr()
+        s0.codes_up, s0.exps_up = s0.codes + gc, s0.exps + ge
         M.w, M.ld_w = _w_ptr(w, id_rows, slots)
         M.expert_n = P["I"]
         M.codes_stride, M.exps_stride = 2 * gc, 2 * ge
         M.bias = P["bias"].data_ptr() if P["bias"] is not None else None
     else:
         s0.glu, s0.n, s0.n_pad = 0, P["H"], dn
-        s0.codes, s0.exps = P["dn"][0].data_ptr(), P["dn_exps"][0].data_ptr()
+        s0.codes, s0.exps = P["dn"].data_ptr(), P["dn_exps"].data_ptr()
         M.expert_k = P["I"]
         M.codes_stride, M.exps_stride = dc, de
-    stream = torch.cuda.current_stream(x2.device)
-    L.stream = stream.cuda_stream
+    L.stream = stream = dev.raw_stream(x2.device)
     lib = _lib.lib()
-    need = lib.dr_moe_workspace_bytes(ctypes.byref(L), ctypes.byref(M))
-    _lib.check(_lib.DR_EINVAL if need < 0 else _lib.DR_OK, "dr_moe_workspace_bytes")
-    if need > 0:
-        ws = linear._workspace(x2.device, stream, need)
+    # the stream's workspace if it has one: a launch that needs more is refused before anything is enqueued
+    ws = linear._WORKSPACE.get((x2.device, stream, "matmul"))
+    if ws is not None:
         L.workspace, L.workspace_bytes = ws.data_ptr(), ws.numel()
-    if route is not None:
-        _lib.check(lib.dr_moe_route_gate_up(ctypes.byref(L), ctypes.byref(M), ctypes.byref(route)), "dr_moe_route_gate_up")
-    else:
-        _lib.check(lib.dr_moe_matmul(ctypes.byref(L), ctypes.byref(M)), "dr_moe_matmul")
+    what = "dr_moe_matmul" if route is None else "dr_moe_route_gate_up"
+
+    def call():
+        if route is None:
+            return lib.dr_moe_matmul(ctypes.byref(L), ctypes.byref(M))
+        return lib.dr_moe_route_gate_up(ctypes.byref(L), ctypes.byref(M), ctypes.byref(route))
+
+    st = call()
+    if st == _lib.DR_EINVAL:
+        need = lib.dr_moe_workspace_bytes(ctypes.byref(L), ctypes.byref(M))
+        if need > 0 and need > L.workspace_bytes:
+            ws = linear._workspace(x2.device, stream, need)
+            L.workspace, L.workspace_bytes = ws.data_ptr(), ws.numel()
+            st = call()
+    _lib.check(st, what)
     return y
 
 
@@ -657,7 +667,7 @@ def _route_args(logits, ids, w, k, kind, bias, ids32, experts, shared, scale, no
     A.scale, A.norm = float(scale), int(bool(norm))
     A.n_group, A.topk_group = ng, tg
     A.slot = -1 if slot is None else int(slot)
-    A.stream = torch.cuda.current_stream(logits.device).cuda_stream
+    A.stream = dev.raw_stream(logits.device)
     return A
 
 
