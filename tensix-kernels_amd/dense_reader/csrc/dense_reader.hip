@@ -47,6 +47,8 @@ constexpr int MAXW = 8;      // wavefronts a workgroup at most (512 threads: up 
 // CU's bytes follow the chunks it has in flight: the gpt-oss down (180 workgroups of 24 chunks) 8.0 -> 6.9 us with 16
 // wavefronts of one or two chunks against 8 of three (12 of two: 7.5 us).
 constexpr int MAXW_DOWN = 16;
+// dr_mfma_moe_down_pairs: K splits at most (its workgroup's LDS, two a CU)
+constexpr int DOWN_SPLITS = 11;
 
 // output columns of a workgroup's tile: 16 (one panel) for a narrow launch (PW = 1), else 32
 template <int PW>
@@ -2094,16 +2096,16 @@ __device__ __forceinline__ void xl_chunk_bfp8_b1(const Args& a, const uint8_t* c
 // bfloat4_b: a step is block k / 128; MFMA D takes k = 32 kq + 8 D + j of the step
 template <int PW, int D = 1>
 __device__ __forceinline__ void xl_chunk_bfp4(const Args& a, const uint8_t* const* cb, const uint8_t* const* eb, int k0,
-                                              int k1, int lane, f32x4 (&acc)[PW][2], uint4* xs, uint32_t xbytes = 0) {
+                                              int k1, int lane, f32x4 (&acc)[PW][2], uint4* xs) {
     static_assert(D == 1 || D == 2, "xl_chunk_bfp4: one or two steps in flight");
     const int ns = (k1 - k0) >> 7;
     if constexpr (D > 1) {
         if (ns % D) {
-            xl_chunk_bfp4<PW, 1>(a, cb, eb, k0, k1, lane, acc, xs, xbytes);
+            xl_chunk_bfp4<PW, 1>(a, cb, eb, k0, k1, lane, acc, xs);
             return;
         }
     }
-    const XStage<16> xst(a, lane, xbytes);
+    const XStage<16> xst(a, lane);
     uint4 cn[D][PW];
     uint32_t en[PW], e[PW];
     auto issue_x = [&](int s) { xst.stage(k0 + 128 * s, xs); };
@@ -2194,6 +2196,78 @@ __device__ __forceinline__ void xl_chunk_bf16(const Args& a, const uint8_t* cons
                 for (int tt = 0; tt < 2; ++tt) acc[q][tt] = mfma(A[u][tt], c[u][q], acc[q][tt]);
     };
     xl_steps<D>(ns, issue_x, issue_c, step);
+}
+
+// The expert gather's down at 32 rows (bfloat4_b): steps [s0, s1) of 128 k in one run, the next step's x staged and its
+// codes and exponents loaded while the current one is decoded. Where a step lies is where(s)'s answer: the k within its
+// weight (kk), the column of x it starts at (xk) and the bytes from expert 0's codes and exponents to its expert's. A
+// wavefront takes one run of consecutive steps, whatever experts it crosses: taken in chunks of 512 k the loop started
+// cold at each, its first loads exposed. (The gate/up, whose run would be 3 steps, is faster in its chunks: 133 us
+// against 143.)
+struct StepAt {
+    int kk, xk;
+    long long co, eo;
+};
+template <int PW, typename F>
+__device__ __forceinline__ void xl_run_bfp4(const Args& a, const uint8_t* const* cb, const uint8_t* const* eb, int s0,
+                                            int s1, int k, int lane, f32x4 (&acc)[PW][2], uint4* xs, uint32_t xbytes,
+                                            F where) {
+    if (s0 >= s1) return;
+    const XStage<16> xst(a, lane, xbytes);
+    uint4 cn[PW];
+    uint32_t en[PW];
+    auto issue = [&](const StepAt& w) {
+        xst.stage(w.xk, xs);
+#pragma unroll
+        for (int q = 0; q < PW; ++q) en[q] = ld_stream4(eb[q] + w.eo + (uint32_t)((w.kk & ~255) + 4 * lane));
+#pragma unroll
+        for (int q = 0; q < PW; ++q) cn[q] = ld_stream16(cb[q] + w.co + (uint32_t)((w.kk >> 7) * 1024 + lane * 16));
+    };
+    auto step = [&](const StepAt& w, auto next) {
+        uint4 c[PW];
+        uint32_t e[PW];
+#pragma unroll
+        for (int q = 0; q < PW; ++q) {
+            c[q] = cn[q];
+            e[q] = en[q] >> (16 * ((w.kk >> 7) & 1));
+        }
+        uint4 A[4][2];  // [D][tt]
+        const int r = lane & 15, kq = lane >> 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) A[j][tt] = x_lds<16>(xs, 16 * tt + r, 4 * kq + j);
+        if (w.kk + 128 > k) {  // (the weight's last step, K not a multiple of 128: the columns past K are zeros)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (w.kk + 8 * (4 * kq + j) >= k) A[j][0] = A[j][1] = make_uint4(0u, 0u, 0u, 0u);
+        }
+        next();
+#pragma unroll
+        for (int q = 0; q < PW; ++q) {
+            const float s0f = __builtin_ldexpf(1.f, (int)(e[q] & 0xFFu) - 133);
+            const float s1f = __builtin_ldexpf(1.f, (int)((e[q] >> 8) & 0xFFu) - 133);
+            const uint4 B0 = b_bfp4<0>(c[q].x, s0f, s1f);
+            const uint4 B1 = b_bfp4<1>(c[q].y, s0f, s1f);
+            const uint4 B2 = b_bfp4<2>(c[q].z, s0f, s1f);
+            const uint4 B3 = b_bfp4<3>(c[q].w, s0f, s1f);
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                acc[q][tt] = mfma(A[0][tt], B0, acc[q][tt]);
+                acc[q][tt] = mfma(A[1][tt], B1, acc[q][tt]);
+                acc[q][tt] = mfma(A[2][tt], B2, acc[q][tt]);
+                acc[q][tt] = mfma(A[3][tt], B3, acc[q][tt]);
+            }
+        }
+    };
+    StepAt w = where(s0);
+    issue(w);
+    for (int s = s0; s + 1 < s1; ++s) {
+        const StepAt n = where(s + 1);
+        step(w, [&] { issue(n); });
+        w = n;
+    }
+    step(w, [] {});
 }
 
 template <int MT, int PW, int FMT, bool ONE>
@@ -2441,10 +2515,9 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
     // memory: one dependent round trip fewer a chunk)
     int idv = -1;
     if constexpr (MOE == DR_MOE_DOWN) idv = lane < a.slots ? moe_id(a, 0, lane) : -1;
-    // 32 rows: x through each wavefront's LDS staging, as the dense 32-row kernel reads it (the same sums; x read in
-    // whole lines). The down's chunk views x from its unit's block on, so its staging may read only up to x's end.
+    // 32 rows of gate/up: x through each wavefront's LDS staging, as the dense 32-row kernel reads it (the same sums;
+    // x read in whole lines)
     constexpr bool XLG = MOE == DR_MOE_GATE_UP_ROWS && MT == 2 && !KB;
-    constexpr bool XLD = MOE == DR_MOE_DOWN_ROWS && MT == 2 && !KB;
     uint4* xs = reinterpret_cast<uint4*>(part) + wave * (XS_BYTES / 16);
     const int ch1 = min((split + 1) * a.cps, a.chunks);
     for (int ch = split * a.cps + wave; ch < ch1; ch += a.waves) {
@@ -2465,12 +2538,7 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
                 cbe[q] = cb[q] + (size_t)e * a.cstride;
                 ebe[q] = eb[q] + (size_t)e * a.estride;
             }
-            if constexpr (XLD) {
-                const uint32_t xb = 2u * (uint32_t)a.ldx * (uint32_t)a.m - 2u * (uint32_t)(s * a.ek);  // (to x's end)
-                xl_chunk_bfp4<PW>(b, cbe, ebe, k0 - s * a.ekp, k1 - s * a.ekp, lane, acc, xs, xb);
-            } else {
-                chunk(b, cbe, ebe, k0 - s * a.ekp, k1 - s * a.ekp);
-            }
+            chunk(b, cbe, ebe, k0 - s * a.ekp, k1 - s * a.ekp);
         } else {
             if constexpr (XLG)
                 xl_chunk_bfp4<PW>(a, cb, eb, k0, k1, lane, acc, xs);
@@ -2478,7 +2546,7 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
                 chunk(a, cb, eb, k0, k1);
         }
     }
-    if constexpr (XLG || XLD) __syncthreads();  // (every wavefront done with its staging before any partial lands on it)
+    if constexpr (XLG) __syncthreads();  // (every wavefront done with its staging before any partial lands on it)
 #pragma unroll
     for (int q = 0; q < PW; ++q)
 #pragma unroll
@@ -2555,6 +2623,62 @@ __global__ __launch_bounds__(512) void dr_mfma_moe_pairs(const MoeArgs a) {
         moe_pair_tiles<2>(a, t0, unit, ex, wave, lane, part);
     else
         moe_pair_tiles<1>(a, t0, unit, ex, wave, lane, part);
+}
+
+// DR_MOE_DOWN_ROWS at 32 rows: two adjacent 32-column tiles a workgroup (the last of an odd count alone), so that the
+// staged x serves both, and the union's steps (its experts' K one after another) shared out evenly over the splits'
+// wavefronts, each one run of them. With a chunk of 512 k at a time over one tile, each wavefront had 2 KB of codes in
+// flight and started cold at every chunk: the gpt-oss shape at 17 and 32 rows took 78 and 86 us, and takes 59 and 64 now
+// (132.7 MB of codes: 2.2 and 2.1 TB/s, the decoding's rate). LDS: the wavefronts' x staging, then the partial sums of
+// the second tile, which meet first, and of the first.
+__global__ __launch_bounds__(512, 4) void dr_mfma_moe_down_pairs(const MoeArgs a) {
+    extern __shared__ float part[];
+    UnionLds* ul = union_lds<DR_MOE_DOWN_ROWS>();
+    moe_union(a, *ul);
+    const SegDev& sg = a.seg[0];
+    const int tp = (a.tiles + 1) / 2, gp = blockIdx.x % tp, split = blockIdx.x / tp;
+    const int t0 = 2 * gp, nt = min(2, a.tiles - t0);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint8_t* cb[4];
+    const uint8_t* eb[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int pan = 2 * (t0 + (nt == 2 ? q >> 1 : 0)) + (q & 1);
+        cb[q] = sg.codes + (size_t)pan * sg.pstride;
+        eb[q] = sg.exps + (size_t)pan * a.ekp;
+    }
+    f32x4 acc[4][2];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) acc[q][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint4* xs = reinterpret_cast<uint4*>(part) + wave * (XS_BYTES / 16);
+    const int per = (a.ek + 127) / 128, ns = ul->count * per;  // steps of an expert, of the union
+    const int w = split * a.waves + wave, W = a.splits * a.waves;
+    xl_run_bfp4<4>(a, cb, eb, (int)((long long)ns * w / W), (int)((long long)ns * (w + 1) / W), a.ek, lane, acc, xs,
+                   2u * (uint32_t)(a.ldx * (a.m - 1) + a.k_pad / a.ekp * a.ek),  // (to the end of x's last row)
+                   [&](int st) {
+                       const int u = st / per, kk = 128 * (st - u * per);
+                       const int e = __builtin_amdgcn_readfirstlane((int)ul->list[u]);
+                       return StepAt{kk, u * a.ek + kk, e * a.cstride, e * a.estride};
+                   });
+    __syncthreads();  // (every wavefront done with its staging before any partial lands on it)
+    const int U = a.waves * 2 * 32 * 16;  // floats from one tile's partials to the next's
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                part[(q >> 1) * U + ((wave * 2 + (q & 1)) * 32 + 16 * tt + 4 * (lane >> 4) + j) * 16 + (lane & 15)] =
+                    acc[q][tt][j];
+    __syncthreads();
+#pragma unroll 1
+    for (int u = nt - 1; u >= 0; --u) {
+        const int nparts = gather_splits<32, 2>(a, t0 + u, split, part + u * U);
+        if (nparts) epilogue<32, 2>(a, sg, t0 + u, part + u * U, nparts, nullptr, nullptr, wave, lane);
+        __syncthreads();  // (the second tile's sums read before the first's land on them)
+    }
 }
 
 // ---- packing ---------------------------------------------------------------------------------------------------------
@@ -3106,7 +3230,7 @@ template <int MT, int PW, int MOE>
 void launch_mfma_moe(const MoeArgs& a, int grid, hipStream_t st) {
     const dim3 b(64 * a.waves);
     size_t lds = (size_t)max(a.waves, a.splits) * PW * 16 * MT * 16 * sizeof(float);
-    if ((MOE == DR_MOE_GATE_UP_ROWS || MOE == DR_MOE_DOWN_ROWS) && MT == 2)
+    if (MOE == DR_MOE_GATE_UP_ROWS && MT == 2)
         lds = max(lds, (size_t)a.waves * XS_BYTES);  // (the x staging)
     if (a.seg[0].fmt == DR_BFP4_KB)
         hipLaunchKernelGGL((dr_mfma_moe<MT, PW, MOE, true>), dim3(grid), b, lds, st, a);
@@ -3150,8 +3274,13 @@ hipError_t launch_moe(const MoeArgs& a, int mode, int rows, int pw, int grid, hi
                         : launch_gemv_moe<2, 2, DR_MOE_DOWN_ROWS>(a, grid, st);
             else if (rows == 16)
                 launch_mfma_moe<1, 2, DR_MOE_DOWN_ROWS>(a, grid, st);
-            else
-                launch_mfma_moe<2, 2, DR_MOE_DOWN_ROWS>(a, grid, st);
+            else if (a.seg[0].fmt == DR_BFP4) {
+                const size_t unit = 2 * 32 * 16 * sizeof(float);  // a tile's partial sums
+                const size_t lds = max((size_t)a.waves * XS_BYTES, (size_t)(a.waves + max(a.waves, a.splits)) * unit);
+                hipLaunchKernelGGL(dr_mfma_moe_down_pairs, dim3(a.pairs), dim3(64 * a.waves), lds, st, a);
+            } else
+                hipLaunchKernelGGL((dr_mfma_moe<2, 2, DR_MOE_DOWN_ROWS, true>), dim3(grid), dim3(64 * a.waves),
+                                   (size_t)max(a.waves, a.splits) * 2 * 32 * 16 * sizeof(float), st, a);
             break;
     }
     return hipGetLastError();
@@ -3906,6 +4035,16 @@ int prepare_moe(const dr_launch* L, const dr_moe* M, MoeArgs& a, int& pw, int& t
         a.ekp = ekp;
         a.seg[0].pstride = (unsigned)((ekp / kblk(DR_BFP4)) * 1024);
         if (ekp % a.kch) plan_chunks(a.k_pad, 256, &a.chunks, &a.kch, &a.waves, &a.splits, &a.cps);  // (a chunk in one unit)
+        // 32 rows of bfloat4_b: tile pairs, in as many splits as keep two workgroups on every CU in one round (45 pairs of
+        // the gpt-oss shape in 11), each wavefront a run of the union's 128-k steps of its own
+        if (mr == 32 && a.seg[0].fmt == DR_BFP4) {
+            const int tp = (a.seg[0].tiles + 1) / 2, most = units * ((a.ek + 127) / 128);
+            a.waves = MAXW;
+            a.splits = std::max(1, std::min({2 * cu_count() / tp, DOWN_SPLITS, (most + MAXW - 1) / MAXW}));
+            a.cps = (a.chunks + a.splits - 1) / a.splits;
+            if (tiles > SPLIT_MAXTILES) a.splits = 1;
+            a.pairs = tp * a.splits;
+        }
         // The GEMV's tile width and K splits (the down modes have no block lists, so they may depend on N): the pair
         // of the lowest cost, ceil(workgroups / CUs) rounds of cps chunks x the width each plus a workgroup's fixed
         // cost (its start, barrier and epilogue: about two 16-column chunks), plus the splits' meeting (about four);
