@@ -1081,39 +1081,62 @@ __device__ __forceinline__ void epilogue(const Args& a, const SegDev& sg, int t,
 // for the expert (the slot's in DR_MOE_GATE_UP; 0 where the row did not choose it in DR_MOE_GATE_UP_ROWS) and writes
 // the unit's columns of y (moe_gu_compute.cpp: the GLU in dest, then times the weight's tile). The tile is PW / 2 gate
 // panels then as many up panels: 32 columns, or 16 in a narrow launch (PW = 2).
+// The rows' routing weights come from cw (moe_coefs) where the kernel found them before its K loop, else from here; a
+// thread's elements are all of one column, whose bias is read once, before the sums.
 template <int ROWS, int PW, int MOE>
 __device__ __forceinline__ void epilogue_moe(const MoeArgs& a, int t, int unit, int ex, const float* part, int nparts,
-                                             float wunit) {
+                                             float wunit, const uint32_t* cw = nullptr) {
     constexpr int TW = 8 * PW, H = PW / 2;
+    static_assert(64 % TW == 0, "epilogue_moe: a thread's elements lie in one column");
     __shared__ float coef[ROWS];
     const int mrows = min(a.m, ROWS);
-    if (threadIdx.x < ROWS) {
-        const int m = threadIdx.x, r = a.row0 + m;
-        float c = 0.f;
-        if (m < mrows) {
-            if (MOE == DR_MOE_GATE_UP) {
-                c = wunit;  // (the slot's weight, read or routed at the workgroup's start)
-            } else if (r < a.id_rows) {
-                for (int j = 0; j < a.slots; ++j)
-                    if (moe_id(a, r, j) == ex) c = bf16_to_f32(a.rw[(size_t)r * a.ld_rw + j]);
-            }
-        }
-        coef[m] = c;
+    const int col = threadIdx.x % TW, oc = t * TW + col;  // the column within the tile, the expert's
+    float gb = 0.f, ub = 0.f;
+    if (a.bias != nullptr && oc < a.en) {
+        gb = bf16_to_f32(a.bias[((size_t)ex * 2 + 0) * a.en + oc]);
+        ub = bf16_to_f32(a.bias[((size_t)ex * 2 + 1) * a.en + oc]);
     }
-    __syncthreads();
+    if (cw == nullptr) {
+        if (threadIdx.x < ROWS) {
+            const int m = threadIdx.x, r = a.row0 + m;
+            float c = 0.f;
+            if (m < mrows) {
+                if (MOE == DR_MOE_GATE_UP) {
+                    c = wunit;  // (the slot's weight, read or routed at the workgroup's start)
+                } else if (r < a.id_rows) {
+                    for (int j = 0; j < a.slots; ++j)
+                        if (moe_id(a, r, j) == ex) c = bf16_to_f32(a.rw[(size_t)r * a.ld_rw + j]);
+                }
+            }
+            coef[m] = c;
+        }
+        __syncthreads();
+    }
     for (int e = threadIdx.x; e < TW * ROWS; e += wg_threads(a)) {
-        const int m = e / TW, col = e % TW;
-        const int oc = t * TW + col;  // the column within the expert's
+        const int m = e / TW;
         if (m >= mrows || oc >= a.en) continue;
         const int cq = col >> 4, cc = col & 15;
         float gsum = sum_parts(0.f, part + (cq * ROWS + m) * 16 + cc, nparts, PW * ROWS * 16);
         float usum = sum_parts(0.f, part + ((H + cq) * ROWS + m) * 16 + cc, nparts, PW * ROWS * 16);
         if (a.bias != nullptr) {
-            gsum += bf16_to_f32(a.bias[((size_t)ex * 2 + 0) * a.en + oc]);
-            usum += bf16_to_f32(a.bias[((size_t)ex * 2 + 1) * a.en + oc]);
+            gsum += gb;
+            usum += ub;
         }
-        const float v = glu(gsum, usum, a.act) * coef[m];
+        const float v = glu(gsum, usum, a.act) * (cw != nullptr ? bf16_to_f32((uint16_t)cw[m]) : coef[m]);
         reinterpret_cast<uint16_t*>(a.y)[(size_t)m * a.ldy + (size_t)unit * a.en + oc] = (uint16_t)f32_to_bf16(v);
+    }
+}
+
+// The rows' routing weights for expert ex, before the K loop: cw[m] the bf16 bits of row row0 + m's, under its slot + 1
+// in the upper half (of several slots with the id the last counts); 0 where the row did not choose it. cw is cleared,
+// and cleared before any thread comes here; the caller's barrier after the K loop shows the result. (In the epilogue
+// the slots' ids and weights were dependent round trips to memory with the workgroup waiting.)
+__device__ __forceinline__ void moe_coefs(const MoeArgs& a, int ex, uint32_t* cw, int rows) {
+    const int n = min(a.m, min(rows, a.id_rows - a.row0)) * a.slots;
+    for (int i = threadIdx.x; i < n; i += wg_threads(a)) {
+        const int m = i / a.slots, j = i - m * a.slots;
+        const uint32_t w = a.rw[(size_t)(a.row0 + m) * a.ld_rw + j];
+        if (moe_id(a, a.row0 + m, j) == ex) atomicMax(&cw[m], (uint32_t)(j + 1) << 16 | w);
     }
 }
 
@@ -2471,21 +2494,18 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
     int t = g - sg.tile_begin;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // the expert gather, as dr_gemv_moe's (the rows modes past two rows)
-    UnionLds* ul = nullptr;
-    if constexpr (MOE == DR_MOE_GATE_UP_ROWS || MOE == DR_MOE_DOWN_ROWS) {
-        ul = union_lds<MOE>();
-        moe_union(a, *ul);
-    }
+    static_assert(MOE == DR_MOE_GATE_UP_ROWS || MOE == DR_MOE_DOWN_ROWS, "dr_mfma_moe: the rows modes");
+    __shared__ uint32_t cw[ROWS];
+    UnionLds* ul = union_lds<MOE>();
+    if (moe_n<MOE>() && threadIdx.x < ROWS) cw[threadIdx.x] = 0u;
+    moe_union(a, *ul);
     int unit = 0, ex = 0;
     if constexpr (moe_n<MOE>()) {
         unit = t / a.tpe;
         t -= unit * a.tpe;
-        ex = MOE == DR_MOE_GATE_UP ? moe_id(a, 0, unit) : (unit < ul->count ? (int)ul->list[unit] : -1);
-        ex = __builtin_amdgcn_readfirstlane(ex);
-        if (ex < 0) {
-            if (MOE == DR_MOE_GATE_UP && split == 0) moe_zero<PW>(a, t, unit);
-            return;
-        }
+        ex = __builtin_amdgcn_readfirstlane(unit < ul->count ? (int)ul->list[unit] : -1);
+        if (ex < 0) return;
+        moe_coefs(a, ex, cw, ROWS);
     }
     const uint8_t* cb[PW];
     const uint8_t* eb[PW];
@@ -2511,10 +2531,6 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
                 mgroup_bfp4<MT, PW>(b, cbx, ebx, gg, lane, acc);
         }
     };
-    // DR_MOE_DOWN: every slot's id, lane j slot j, read once (a chunk then takes its unit's id from a lane, not from
-    // memory: one dependent round trip fewer a chunk)
-    int idv = -1;
-    if constexpr (MOE == DR_MOE_DOWN) idv = lane < a.slots ? moe_id(a, 0, lane) : -1;
     // 32 rows of gate/up: x through each wavefront's LDS staging, as the dense 32-row kernel reads it (the same sums;
     // x read in whole lines)
     constexpr bool XLG = MOE == DR_MOE_GATE_UP_ROWS && MT == 2 && !KB;
@@ -2524,8 +2540,7 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
         const int k0 = ch * a.kch, k1 = min(k0 + a.kch, a.k_pad);
         if constexpr (moe_k<MOE>()) {
             const int s = __builtin_amdgcn_readfirstlane(k0 / a.ekp);
-            int e = MOE == DR_MOE_DOWN ? __builtin_amdgcn_readlane(idv, s) : (s < ul->count ? (int)ul->list[s] : -1);
-            e = __builtin_amdgcn_readfirstlane(e);
+            const int e = __builtin_amdgcn_readfirstlane(s < ul->count ? (int)ul->list[s] : -1);
             if (e < 0) continue;
             Args b = a;  // (the chunk's view of x: the unit's block)
             b.x = a.x + (size_t)s * a.ek;
@@ -2558,7 +2573,7 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
     const int nparts = gather_splits<ROWS, PW>(a, g, split, part);
     if (!nparts) return;
     if constexpr (moe_n<MOE>())
-        epilogue_moe<ROWS, PW, MOE>(a, t, unit, ex, part, nparts, 0.f);
+        epilogue_moe<ROWS, PW, MOE>(a, t, unit, ex, part, nparts, 0.f, cw);
     else
         epilogue<ROWS, PW>(a, sg, t, part, nparts, tval, tkey, wave, lane);
 }
@@ -2569,7 +2584,7 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
 // the same order as in dr_mfma_moe<2, 4> (xl_chunk_bfp4 over more panels), so the results do not change.
 template <int NT>
 __device__ __forceinline__ void moe_pair_tiles(const MoeArgs& a, int t0, int unit, int ex, int wave, int lane,
-                                               float* part) {
+                                               float* part, const uint32_t* cw) {
     constexpr int PW = 4 * NT, ROWS = 32;
     const SegDev& sg = a.seg[0];
     const uint8_t* cb[PW];
@@ -2606,23 +2621,26 @@ __device__ __forceinline__ void moe_pair_tiles(const MoeArgs& a, int t0, int uni
                 for (int j = 0; j < 4; ++j)
                     part[((wave * 4 + q) * ROWS + 16 * tt + 4 * (lane >> 4) + j) * 16 + (lane & 15)] = acc[4 * u + q][tt][j];
         __syncthreads();
-        epilogue_moe<ROWS, 4, DR_MOE_GATE_UP_ROWS>(a, t0 + u, unit, ex, part, a.waves, 0.f);
+        epilogue_moe<ROWS, 4, DR_MOE_GATE_UP_ROWS>(a, t0 + u, unit, ex, part, a.waves, 0.f, cw);
     }
 }
 
 __global__ __launch_bounds__(512) void dr_mfma_moe_pairs(const MoeArgs a) {
     extern __shared__ float part[];  // the x staging during the K loop; then one tile's [W][4][32][16]
+    __shared__ uint32_t cw[32];
     UnionLds* ul = union_lds<DR_MOE_GATE_UP_ROWS>();
+    if (threadIdx.x < 32) cw[threadIdx.x] = 0u;
     moe_union(a, *ul);
     const int tp2 = (a.tpe + 1) / 2;
     const int unit = blockIdx.x / tp2, t0 = 2 * (blockIdx.x - unit * tp2);
     const int ex = __builtin_amdgcn_readfirstlane(unit < ul->count ? (int)ul->list[unit] : -1);
     if (ex < 0) return;
+    moe_coefs(a, ex, cw, 32);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (a.tpe - t0 >= 2)
-        moe_pair_tiles<2>(a, t0, unit, ex, wave, lane, part);
+        moe_pair_tiles<2>(a, t0, unit, ex, wave, lane, part, cw);
     else
-        moe_pair_tiles<1>(a, t0, unit, ex, wave, lane, part);
+        moe_pair_tiles<1>(a, t0, unit, ex, wave, lane, part, cw);
 }
 
 // DR_MOE_DOWN_ROWS at 32 rows: two adjacent 32-column tiles a workgroup (the last of an odd count alone), so that the
@@ -4030,6 +4048,16 @@ int prepare_moe(const dr_launch* L, const dr_moe* M, MoeArgs& a, int& pw, int& t
         tiles = units * a.tpe;
         a.seg[0].tiles = tiles;
         a.tiles = tiles;
+        // The MFMA rows, more workgroups than one round of 8 wavefronts each (two on a CU at 16 rows, one at 32, by
+        // registers): 4 wavefronts, each a quarter of K in one run, so that one workgroup's start and epilogue pass
+        // under another's K loop. 12 chunks over 8 wavefronts left half of them idle for half of it too. (The gpt-oss
+        // gate/up at 3, 8, 16, 17 and 32 rows 38.7, 58.7, 87.3, 116, 126 us in 8 wavefronts, 33.7, 50.3, 75.3, 90.0,
+        // 95.5 in 4. In one round 8 are better: 32 experts of 2048 x 768, top 1, at 17 rows 18.5 us against 20.1.)
+        const int wgs = mr == 32 && s0.fmt == DR_BFP4 ? units * ((a.tpe + 1) / 2) : tiles;
+        if (mr >= 16 && !DR_CHUNK_K && a.splits == 1 && a.chunks > 4 && wgs > (mr == 32 ? 1 : 2) * cu_count()) {
+            plan_chunks(a.k_pad, (a.k_pad + 4 * KALIGN - 1) / (4 * KALIGN) * KALIGN, &a.chunks, &a.kch, &a.waves,
+                        &a.splits, &a.cps);
+        }
     } else {
         a.ek = M->expert_k;
         a.ekp = ekp;
