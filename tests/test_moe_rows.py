@@ -1,9 +1,10 @@
-"""The MoE down over 17 to 32 rows of bfloat4_b experts (dr_mfma_moe_down_pairs: tiles in pairs, the union's 128-k
-steps shared out over the splits' wavefronts), at the shapes where its plan has an edge: one tile and an odd count of
-tiles (H), an expert's K of a part of a step, of a step, of one more than a step and of many (I), unions of one expert
-(fewer steps than wavefronts) up to all of them, one split and several. Against the oracle's float64 sum over h as the
+"""The MoE over 3 to 32 rows at the edges of its plans. test_down_rows: dr_mfma_moe_down_pairs (17 to 32 rows of
+bfloat4_b experts: tiles in pairs, the union's 128-k steps shared out over the splits' wavefronts), one tile and an odd
+count of tiles (H), an expert's K of a part of a step, of a step, of one more than a step and of many (I), unions of one
+expert (fewer steps than wavefronts) up to all of them, one split and several. Against the float64 sum over h as the
 device holds it, so the bound is derived: y is a bf16 rounding (2^-9 of the value) of float32 sums of exact products,
-whose order costs at most n 2^-24 of the sum of the products' magnitudes, n their count."""
+whose order costs at most n 2^-24 of the sum of the products' magnitudes, n their count. test_gate_up_rows: the same
+bound carried through the activation."""
 
 import pytest
 import torch
@@ -11,6 +12,7 @@ import torch
 from common.testing import same
 from moe import moe8
 from oracle import dense_oracle as O
+from oracle import moe_oracle as MO
 
 pytestmark = pytest.mark.gpu
 
@@ -51,3 +53,50 @@ def test_down_rows(device, E, k, H, I, R):
     bound = ref.abs() * 2.0 ** -8 + mag * (len(u) * I * 2.0 ** -24) + 1e-30
     assert bool((err <= bound).all()), f"worst {float((err / bound).max()):.3f} of its bound"
     assert not yd[R:].any(), "rows past R"
+
+
+# more workgroups than one round of 8 wavefronts takes: 4 wavefronts of one run of K each (6 and 9 groups of 256 k:
+# uneven runs, a wavefront without one), tiles in pairs and an odd one, a row's ids twice the same (the last counts)
+@pytest.mark.parametrize("E, k, H, I, R, kblock", [
+    (16, 4, 1312, 1056, 32, False),
+    (16, 4, 1504, 1056, 17, True),
+    (32, 4, 2080, 544, 16, False),
+    (32, 8, 1312, 608, 7, True),
+])
+def test_gate_up_rows(device, E, k, H, I, R, kblock):
+    print(f"case E {E} k {k} H {H} I {I} rows {R} kblock {kblock}", flush=True)
+    g = torch.Generator().manual_seed(H + I)
+
+    def grid(w):
+        return torch.from_numpy(MO.held_kblock(w.numpy()) if kblock else O.held(w, "bfp4")).float()
+
+    gu = torch.stack([grid(torch.randn(H, 2 * I, generator=g) * H ** -0.5) for _ in range(E)])
+    gb = torch.randn(E, 2 * I, generator=g).to(BF)
+    P = moe8.pack(device, gu.to(BF), torch.zeros(E, I, H, dtype=BF), kblock=kblock, gu_bias=gb)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(R)])
+    ids[0, 1] = ids[0, 0]
+    w = torch.softmax(torch.randn(R, k, generator=g), 1).to(BF)
+    tid = ids.to(torch.int16).reshape(1, 1, R, k).to(device.torch)
+    x = torch.randn(R, H, generator=g).to(BF)
+    tx, tw = x.reshape(1, 1, R, H).to(device.torch), w.reshape(1, 1, R, k).to(device.torch)
+    h = moe8.gate_up_rows(tx, P, tid, tw, k, R, loaders=2)
+    same("h repeated", moe8.gate_up_rows(tx, P, tid, tw, k, R, loaders=2).cpu(), h.cpu())
+    u = sorted(set(ids.flatten().tolist()))
+    ref = torch.zeros(R, len(u) * I, dtype=torch.float64)
+    tol = torch.zeros_like(ref)
+    for q, e in enumerate(u):
+        c = torch.zeros(R, dtype=torch.float64)
+        for r in range(R):
+            for j in range(k):
+                if ids[r, j] == e:
+                    c[r] = w[r, j].double()
+        z = x.double() @ gu[e].double() + gb[e].double()
+        z_err = (x.double().abs() @ gu[e].double().abs() + gb[e].double().abs()) * (H * 2.0 ** -24)
+        up, gate, ue, ge = z[:, :I], z[:, I:], z_err[:, :I], z_err[:, I:]  # ([up | gate], as the oracle's layer)
+        cols = slice(q * I, (q + 1) * I)
+        ref[:, cols] = gate * torch.sigmoid(gate) * up * c[:, None]
+        # (silu's slope is at most 1.1; its float32 evaluation within 2^-18 of its argument)
+        tol[:, cols] = ((1.1 * ge + gate.abs() * 2.0 ** -18) * up.abs() + gate.abs() * ue) * c[:, None]
+    hd = h.cpu().double().reshape(-1, h.shape[-1])[:R, :len(u) * I]
+    err, bound = (hd - ref).abs(), ref.abs() * 2.0 ** -8 + 2 * tol + 1e-30
+    assert bool((err <= bound).all()), f"worst {float((err / bound).max()):.3f} of its bound"
