@@ -113,6 +113,8 @@ struct MoeArgs : Args {
     const uint16_t* rw;  // routing weights [id_rows][ld_rw] bf16
     int ld_rw;
     int en, tpe;         // gate/up modes: an expert's output columns, its 32-column tiles
+    int chains;          // the MFMA rows modes: a tile's partial sums, chain c the chunks c, c + chains, ... in order;
+                         // wavefront w sums chains w, w + waves, ... (chains > waves: gate/up, unsplit)
     int ek, ekp;         // down modes: an expert's rows (x's block width) and the rows packed (a multiple of 256)
     long long cstride, estride;  // bytes from one expert's codes / exponents to the next
     const uint16_t* bias;        // gate/up modes: [experts][2][en] bf16 (gate, up) or null
@@ -1083,9 +1085,11 @@ __device__ __forceinline__ void epilogue(const Args& a, const SegDev& sg, int t,
 // panels then as many up panels: 32 columns, or 16 in a narrow launch (PW = 2).
 // The rows' routing weights come from cw (moe_coefs) where the kernel found them before its K loop, else from here; a
 // thread's elements are all of one column, whose bias is read once, before the sums.
+// run: the sums that part's are added to ([PW][ROWS][16]; null: zeros).
 template <int ROWS, int PW, int MOE>
 __device__ __forceinline__ void epilogue_moe(const MoeArgs& a, int t, int unit, int ex, const float* part, int nparts,
-                                             float wunit, const uint32_t* cw = nullptr) {
+                                             float wunit, const uint32_t* cw = nullptr,
+                                             const float* run = nullptr) {
     constexpr int TW = 8 * PW, H = PW / 2;
     static_assert(64 % TW == 0, "epilogue_moe: a thread's elements lie in one column");
     __shared__ float coef[ROWS];
@@ -1115,9 +1119,9 @@ __device__ __forceinline__ void epilogue_moe(const MoeArgs& a, int t, int unit, 
     for (int e = threadIdx.x; e < TW * ROWS; e += wg_threads(a)) {
         const int m = e / TW;
         if (m >= mrows || oc >= a.en) continue;
-        const int cq = col >> 4, cc = col & 15;
-        float gsum = sum_parts(0.f, part + (cq * ROWS + m) * 16 + cc, nparts, PW * ROWS * 16);
-        float usum = sum_parts(0.f, part + ((H + cq) * ROWS + m) * 16 + cc, nparts, PW * ROWS * 16);
+        const int cq = col >> 4, cc = col & 15, ig = (cq * ROWS + m) * 16 + cc, iu = ((H + cq) * ROWS + m) * 16 + cc;
+        float gsum = sum_parts(run != nullptr ? run[ig] : 0.f, part + ig, nparts, PW * ROWS * 16);
+        float usum = sum_parts(run != nullptr ? run[iu] : 0.f, part + iu, nparts, PW * ROWS * 16);
         if (a.bias != nullptr) {
             gsum += gb;
             usum += ub;
@@ -2225,16 +2229,19 @@ __device__ __forceinline__ void xl_chunk_bf16(const Args& a, const uint8_t* cons
 // codes and exponents loaded while the current one is decoded. Where a step lies is where(s)'s answer: the k within its
 // weight (kk), the column of x it starts at (xk) and the bytes from expert 0's codes and exponents to its expert's. A
 // wavefront takes one run of consecutive steps, whatever experts it crosses: taken in chunks of 512 k the loop started
-// cold at each, its first loads exposed. (The gate/up, whose run would be 3 steps, is faster in its chunks: 133 us
-// against 143.)
+// cold at each, its first loads exposed. The gate/up takes a wavefront's chains of chunks in one run the same way
+// (moe_pair_tiles), with between() after step `last` of the first chain.
 struct StepAt {
     int kk, xk;
     long long co, eo;
 };
-template <int PW, typename F>
+struct NoBetween {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <int PW, typename F, typename G = NoBetween>
 __device__ __forceinline__ void xl_run_bfp4(const Args& a, const uint8_t* const* cb, const uint8_t* const* eb, int s0,
                                             int s1, int k, int lane, f32x4 (&acc)[PW][2], uint4* xs, uint32_t xbytes,
-                                            F where) {
+                                            F where, int last = -1, G between = G{}) {
     if (s0 >= s1) return;
     const XStage<16> xst(a, lane, xbytes);
     uint4 cn[PW];
@@ -2288,9 +2295,19 @@ __device__ __forceinline__ void xl_run_bfp4(const Args& a, const uint8_t* const*
     for (int s = s0; s + 1 < s1; ++s) {
         const StepAt n = where(s + 1);
         step(w, [&] { issue(n); });
+        if (s == last) between();
         w = n;
     }
     step(w, [] {});
+    if (s1 - 1 == last) between();
+}
+
+// the workgroup's barrier with the wavefronts' LDS instructions done, and their loads from memory still in flight
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 }
 
 template <int MT, int PW, int FMT, bool ONE>
@@ -2518,11 +2535,7 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
         }
     }
 
-    f32x4 acc[PW][MT];  // this wavefront's sums over its chunks, in order
-#pragma unroll
-    for (int q = 0; q < PW; ++q)
-#pragma unroll
-        for (int tt = 0; tt < MT; ++tt) acc[q][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[PW][MT];  // this wavefront's sums over a chain's chunks, in order
     auto chunk = [&](const Args& b, const uint8_t* const* cbx, const uint8_t* const* ebx, int k0, int k1) {
         for (int gg = k0 >> 8; gg < (k1 >> 8); ++gg) {
             if constexpr (KB)
@@ -2536,41 +2549,51 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
     constexpr bool XLG = MOE == DR_MOE_GATE_UP_ROWS && MT == 2 && !KB;
     uint4* xs = reinterpret_cast<uint4*>(part) + wave * (XS_BYTES / 16);
     const int ch1 = min((split + 1) * a.cps, a.chunks);
-    for (int ch = split * a.cps + wave; ch < ch1; ch += a.waves) {
-        const int k0 = ch * a.kch, k1 = min(k0 + a.kch, a.k_pad);
-        if constexpr (moe_k<MOE>()) {
-            const int s = __builtin_amdgcn_readfirstlane(k0 / a.ekp);
-            const int e = __builtin_amdgcn_readfirstlane(s < ul->count ? (int)ul->list[s] : -1);
-            if (e < 0) continue;
-            Args b = a;  // (the chunk's view of x: the unit's block)
-            b.x = a.x + (size_t)s * a.ek;
-            b.k = a.ek;
-            b.k_pad = a.ekp;
-            const uint8_t* cbe[PW];
-            const uint8_t* ebe[PW];
+    const int nch = moe_n<MOE>() ? a.chains : a.waves;  // (the down modes: a chain a wavefront)
+    int c = wave;
+    do {
 #pragma unroll
-            for (int q = 0; q < PW; ++q) {
-                cbe[q] = cb[q] + (size_t)e * a.cstride;
-                ebe[q] = eb[q] + (size_t)e * a.estride;
+        for (int q = 0; q < PW; ++q)
+#pragma unroll
+            for (int tt = 0; tt < MT; ++tt) acc[q][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int ch = split * a.cps + c; ch < ch1; ch += nch) {
+            const int k0 = ch * a.kch, k1 = min(k0 + a.kch, a.k_pad);
+            if constexpr (moe_k<MOE>()) {
+                const int s = __builtin_amdgcn_readfirstlane(k0 / a.ekp);
+                const int e = __builtin_amdgcn_readfirstlane(s < ul->count ? (int)ul->list[s] : -1);
+                if (e < 0) continue;
+                Args b = a;  // (the chunk's view of x: the unit's block)
+                b.x = a.x + (size_t)s * a.ek;
+                b.k = a.ek;
+                b.k_pad = a.ekp;
+                const uint8_t* cbe[PW];
+                const uint8_t* ebe[PW];
+    #pragma unroll
+                for (int q = 0; q < PW; ++q) {
+                    cbe[q] = cb[q] + (size_t)e * a.cstride;
+                    ebe[q] = eb[q] + (size_t)e * a.estride;
+                }
+                chunk(b, cbe, ebe, k0 - s * a.ekp, k1 - s * a.ekp);
+            } else {
+                if constexpr (XLG)
+                    xl_chunk_bfp4<PW>(a, cb, eb, k0, k1, lane, acc, xs);
+                else
+                    chunk(a, cb, eb, k0, k1);
             }
-            chunk(b, cbe, ebe, k0 - s * a.ekp, k1 - s * a.ekp);
-        } else {
-            if constexpr (XLG)
-                xl_chunk_bfp4<PW>(a, cb, eb, k0, k1, lane, acc, xs);
-            else
-                chunk(a, cb, eb, k0, k1);
         }
-    }
-    if constexpr (XLG) __syncthreads();  // (every wavefront done with its staging before any partial lands on it)
+        if constexpr (XLG) __syncthreads();  // (every wavefront, one chain each, done with its staging before any
+                                             // partial lands on it)
 #pragma unroll
-    for (int q = 0; q < PW; ++q)
+        for (int q = 0; q < PW; ++q)
 #pragma unroll
-        for (int tt = 0; tt < MT; ++tt)
+            for (int tt = 0; tt < MT; ++tt)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                part[((wave * PW + q) * ROWS + 16 * tt + 4 * (lane >> 4) + j) * 16 + (lane & 15)] = acc[q][tt][j];
+                for (int j = 0; j < 4; ++j)
+                    part[((c * PW + q) * ROWS + 16 * tt + 4 * (lane >> 4) + j) * 16 + (lane & 15)] = acc[q][tt][j];
+        c += a.waves;
+    } while (moe_n<MOE>() && c < nch);
     __syncthreads();
-    const int nparts = gather_splits<ROWS, PW>(a, g, split, part);
+    const int nparts = a.splits == 1 ? a.chains : gather_splits<ROWS, PW>(a, g, split, part);
     if (!nparts) return;
     if constexpr (moe_n<MOE>())
         epilogue_moe<ROWS, PW, MOE>(a, t, unit, ex, part, nparts, 0.f, cw);
@@ -2579,10 +2602,12 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
 }
 
 // DR_MOE_GATE_UP_ROWS at 32 rows: two adjacent 32-column tiles of one unit's expert a workgroup, so the wavefronts'
-// staged x serves both (the unit's tiles in pairs, the last of an odd count alone): the gpt-oss gate/up at 17, 24 and
-// 32 rows 122, 135, 148 -> 107, 125, 128 us. Each tile's panels are summed by the same lanes, steps and wavefronts in
-// the same order as in dr_mfma_moe<2, 4> (xl_chunk_bfp4 over more panels), so the results do not change.
-template <int NT>
+// staged x serves both (the unit's tiles in pairs, the last of an odd count alone). Each tile's panels are summed in the
+// chains and steps of dr_mfma_moe<2, 4> (xl_chunk_bfp4 over more panels), so the results do not depend on the pairing.
+// TWO: four wavefronts for five to eight chains (prepare_moe says when). A wavefront takes its two chains' steps in one
+// run, the second's loads in flight across the first's end, where the workgroup adds the first four chains' sums up
+// (in LDS after the staging); the last chains' are added to those, so the sums are those of a wavefront a chain.
+template <int NT, bool TWO>
 __device__ __forceinline__ void moe_pair_tiles(const MoeArgs& a, int t0, int unit, int ex, int wave, int lane,
                                                float* part, const uint32_t* cw) {
     constexpr int PW = 4 * NT, ROWS = 32;
@@ -2601,32 +2626,79 @@ __device__ __forceinline__ void moe_pair_tiles(const MoeArgs& a, int t0, int uni
         }
     }
     f32x4 acc[PW][2];
+    auto clear = [&] {
 #pragma unroll
-    for (int q = 0; q < PW; ++q)
+        for (int q = 0; q < PW; ++q)
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) acc[q][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    uint4* xs = reinterpret_cast<uint4*>(part) + wave * (XS_BYTES / 16);
-    for (int ch = wave; ch < a.chunks; ch += a.waves) {
-        const int k0 = ch * a.kch, k1 = min(k0 + a.kch, a.k_pad);
-        xl_chunk_bfp4<PW>(a, cb, eb, k0, k1, lane, acc, xs);
-    }
-#pragma unroll
-    for (int u = 0; u < NT; ++u) {
-        __syncthreads();  // (the staging, or the previous tile's epilogue, done with part)
+            for (int tt = 0; tt < 2; ++tt) acc[q][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto store = [&](float* to, int u) {  // tile u's sums of this wavefront
+        const int l = (int)opaque((uint32_t)lane);  // (addresses made here, not held across the K loop)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    part[((wave * 4 + q) * ROWS + 16 * tt + 4 * (lane >> 4) + j) * 16 + (lane & 15)] = acc[4 * u + q][tt][j];
+                    to[((wave * 4 + q) * ROWS + 16 * tt + 4 * (l >> 4) + j) * 16 + (l & 15)] = acc[4 * u + q][tt][j];
+    };
+    clear();
+    uint4* xs = reinterpret_cast<uint4*>(part) + wave * (XS_BYTES / 16);
+    constexpr int E = 4 * ROWS * 16;  // a tile's sums
+    float* meet = part + 4 * (XS_BYTES / 4);  // TWO: a tile's sums of each wavefront, and the first of two tiles' total
+    int nparts = a.waves;
+    if constexpr (TWO) {
+        const int per = a.kch >> 7, all = (a.k + 127) >> 7;  // steps of a chunk, of K
+        auto steps = [&](int c) {  // of chain c: whole chunks, but for K's last
+            int n = 0;
+            for (int ch = c; c < a.chains && ch < a.chunks; ch += a.chains) n += min(per, all - ch * per);
+            return n;
+        };
+        const int n1 = steps(wave), n2 = steps(wave + 4);
+        xl_run_bfp4<PW>(
+            a, cb, eb, 0, n1 + n2, a.k, lane, acc, xs, 0u,
+            [&](int s) {
+                const int c = s < n1 ? wave : wave + 4, i = s < n1 ? s : s - n1, j = __builtin_amdgcn_readfirstlane(i / per);
+                const int kk = 128 * ((c + a.chains * j) * per + i - j * per);
+                return StepAt{kk, kk, 0, 0};
+            },
+            n1 - 1,
+            [&] {
+#pragma unroll
+                for (int u = 0; u < NT; ++u) {
+                    if (u) lds_barrier();  // (the tile before read)
+                    store(meet, u);
+                    lds_barrier();
+                    float* to = meet + (NT == 2 && u == 0 ? 4 * E : 0);
+#pragma unroll
+                    for (int i = 0; i < E / 256; ++i) {
+                        const int e = threadIdx.x + 256 * i;
+                        to[e] = sum_parts(0.f, meet + e, 4, E);
+                    }
+                }
+                clear();
+            });
+        nparts = a.chains - 4;
+    } else {
+        for (int ch = wave; ch < a.chunks; ch += a.waves) {
+            const int k0 = ch * a.kch, k1 = min(k0 + a.kch, a.k_pad);
+            xl_chunk_bfp4<PW>(a, cb, eb, k0, k1, lane, acc, xs);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+        __syncthreads();  // (the staging, or the previous tile's epilogue, done with part)
+        store(part, u);
         __syncthreads();
-        epilogue_moe<ROWS, 4, DR_MOE_GATE_UP_ROWS>(a, t0 + u, unit, ex, part, a.waves, 0.f, cw);
+        epilogue_moe<ROWS, 4, DR_MOE_GATE_UP_ROWS>(a, t0 + u, unit, ex, part, nparts, 0.f, cw,
+                                                    !TWO ? nullptr : meet + (NT == 2 && u == 0 ? 4 * E : 0));
     }
 }
 
-__global__ __launch_bounds__(512) void dr_mfma_moe_pairs(const MoeArgs a) {
-    extern __shared__ float part[];  // the x staging during the K loop; then one tile's [W][4][32][16]
+template <bool TWO>
+__global__ __launch_bounds__(TWO ? 256 : 512, 2) void dr_mfma_moe_pairs(const MoeArgs a) {
+    extern __shared__ float part[];  // the x staging during the K loop (TWO: and [5][4][32][16] after it); then one
+                                     // tile's [W][4][32][16]
     __shared__ uint32_t cw[32];
     UnionLds* ul = union_lds<DR_MOE_GATE_UP_ROWS>();
     if (threadIdx.x < 32) cw[threadIdx.x] = 0u;
@@ -2638,9 +2710,9 @@ __global__ __launch_bounds__(512) void dr_mfma_moe_pairs(const MoeArgs a) {
     moe_coefs(a, ex, cw, 32);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (a.tpe - t0 >= 2)
-        moe_pair_tiles<2>(a, t0, unit, ex, wave, lane, part, cw);
+        moe_pair_tiles<2, TWO>(a, t0, unit, ex, wave, lane, part, cw);
     else
-        moe_pair_tiles<1>(a, t0, unit, ex, wave, lane, part, cw);
+        moe_pair_tiles<1, TWO>(a, t0, unit, ex, wave, lane, part, cw);
 }
 
 // DR_MOE_DOWN_ROWS at 32 rows: two adjacent 32-column tiles a workgroup (the last of an odd count alone), so that the
@@ -2676,7 +2748,7 @@ __global__ __launch_bounds__(512, 4) void dr_mfma_moe_down_pairs(const MoeArgs a
     xl_run_bfp4<4>(a, cb, eb, (int)((long long)ns * w / W), (int)((long long)ns * (w + 1) / W), a.ek, lane, acc, xs,
                    2u * (uint32_t)(a.ldx * (a.m - 1) + a.k_pad / a.ekp * a.ek),  // (to the end of x's last row)
                    [&](int st) {
-                       const int u = st / per, kk = 128 * (st - u * per);
+                       const int u = __builtin_amdgcn_readfirstlane(st / per), kk = 128 * (st - u * per);
                        const int e = __builtin_amdgcn_readfirstlane((int)ul->list[u]);
                        return StepAt{kk, u * a.ek + kk, e * a.cstride, e * a.estride};
                    });
@@ -3247,7 +3319,7 @@ void launch_gemv_moe(const MoeArgs& a, int grid, hipStream_t st) {
 template <int MT, int PW, int MOE>
 void launch_mfma_moe(const MoeArgs& a, int grid, hipStream_t st) {
     const dim3 b(64 * a.waves);
-    size_t lds = (size_t)max(a.waves, a.splits) * PW * 16 * MT * 16 * sizeof(float);
+    size_t lds = (size_t)max(a.chains, a.splits) * PW * 16 * MT * 16 * sizeof(float);
     if (MOE == DR_MOE_GATE_UP_ROWS && MT == 2)
         lds = max(lds, (size_t)a.waves * XS_BYTES);  // (the x staging)
     if (a.seg[0].fmt == DR_BFP4_KB)
@@ -3277,9 +3349,12 @@ hipError_t launch_moe(const MoeArgs& a, int mode, int rows, int pw, int grid, hi
             else if (rows == 16)
                 launch_mfma_moe<1, 4, DR_MOE_GATE_UP_ROWS>(a, grid, st);
             else if (a.seg[0].fmt != DR_BFP4_KB && a.splits == 1) {
-                const size_t lds = max((size_t)a.waves * XS_BYTES, (size_t)a.waves * 4 * 32 * 16 * sizeof(float));
-                hipLaunchKernelGGL(dr_mfma_moe_pairs, dim3(a.tiles / a.tpe * ((a.tpe + 1) / 2)), dim3(64 * a.waves), lds,
-                                   st, a);
+                const dim3 grid(a.tiles / a.tpe * ((a.tpe + 1) / 2)), b(64 * a.waves);
+                const size_t sums = (size_t)a.waves * 4 * 32 * 16 * sizeof(float), xs = (size_t)a.waves * XS_BYTES;
+                if (a.chains > a.waves)
+                    hipLaunchKernelGGL(dr_mfma_moe_pairs<true>, grid, b, xs + sums / 4 * 5, st, a);
+                else
+                    hipLaunchKernelGGL(dr_mfma_moe_pairs<false>, grid, b, max(xs, sums), st, a);
             } else
                 launch_mfma_moe<2, 4, DR_MOE_GATE_UP_ROWS>(a, grid, st);
             break;
@@ -3298,7 +3373,7 @@ hipError_t launch_moe(const MoeArgs& a, int mode, int rows, int pw, int grid, hi
                 hipLaunchKernelGGL(dr_mfma_moe_down_pairs, dim3(a.pairs), dim3(64 * a.waves), lds, st, a);
             } else
                 hipLaunchKernelGGL((dr_mfma_moe<2, 2, DR_MOE_DOWN_ROWS, true>), dim3(grid), dim3(64 * a.waves),
-                                   (size_t)max(a.waves, a.splits) * 2 * 32 * 16 * sizeof(float), st, a);
+                                   (size_t)max(a.chains, a.splits) * 2 * 32 * 16 * sizeof(float), st, a);
             break;
     }
     return hipGetLastError();
@@ -4048,16 +4123,6 @@ int prepare_moe(const dr_launch* L, const dr_moe* M, MoeArgs& a, int& pw, int& t
         tiles = units * a.tpe;
         a.seg[0].tiles = tiles;
         a.tiles = tiles;
-        // The MFMA rows, more workgroups than one round of 8 wavefronts each (two on a CU at 16 rows, one at 32, by
-        // registers): 4 wavefronts, each a quarter of K in one run, so that one workgroup's start and epilogue pass
-        // under another's K loop. 12 chunks over 8 wavefronts left half of them idle for half of it too. (The gpt-oss
-        // gate/up at 3, 8, 16, 17 and 32 rows 38.7, 58.7, 87.3, 116, 126 us in 8 wavefronts, 33.7, 50.3, 75.3, 90.0,
-        // 95.5 in 4. In one round 8 are better: 32 experts of 2048 x 768, top 1, at 17 rows 18.5 us against 20.1.)
-        const int wgs = mr == 32 && s0.fmt == DR_BFP4 ? units * ((a.tpe + 1) / 2) : tiles;
-        if (mr >= 16 && !DR_CHUNK_K && a.splits == 1 && a.chunks > 4 && wgs > (mr == 32 ? 1 : 2) * cu_count()) {
-            plan_chunks(a.k_pad, (a.k_pad + 4 * KALIGN - 1) / (4 * KALIGN) * KALIGN, &a.chunks, &a.kch, &a.waves,
-                        &a.splits, &a.cps);
-        }
     } else {
         a.ek = M->expert_k;
         a.ekp = ekp;
@@ -4109,6 +4174,16 @@ int prepare_moe(const dr_launch* L, const dr_moe* M, MoeArgs& a, int& pw, int& t
         }
     }
     limit_splits(a);
+    a.chains = a.waves;
+    // The MFMA rows of gate/up, more workgroups than one round of 8 wavefronts each (two on a CU at 16 rows, one at 32,
+    // by registers): 4 wavefronts of two chains of chunks each, so that one workgroup's start and epilogue pass under
+    // another's K loop. 12 chunks over 8 wavefronts left half of them idle for half of it too. The chains and their order
+    // are those of a wavefront each, so a row's bits do not depend on the choice. (The gpt-oss gate/up at 3, 8, 16, 17
+    // and 32 rows 40, 65, 88, 110, 134 us in 8 wavefronts, 36, 55, 76, 89, 111 in 4.)
+    if (nmode && mr >= 16 && a.splits == 1 && a.waves > 4) {
+        const int wgs = mr == 32 && s0.fmt == DR_BFP4 ? units * ((a.tpe + 1) / 2) : tiles;
+        if (wgs > (mr == 32 ? 1 : 2) * cu_count()) a.waves = 4;
+    }
     return DR_OK;
 }
 

@@ -100,3 +100,29 @@ def test_gate_up_rows(device, E, k, H, I, R, kblock):
     hd = h.cpu().double().reshape(-1, h.shape[-1])[:R, :len(u) * I]
     err, bound = (hd - ref).abs(), ref.abs() * 2.0 ** -8 + 2 * tol + 1e-30
     assert bool((err <= bound).all()), f"worst {float((err / bound).max()):.3f} of its bound"
+
+
+# The wavefronts of a gate/up workgroup follow the launch's size (four with two chains of chunks each, or eight), its sums
+# do not: the first columns of wide experts, whose launch takes four, against the same columns packed alone, bit for bit.
+# The two halves of K nearly cancel, so that sums in another order differ in most values.
+@pytest.mark.parametrize("H", [1312, 2080, 4160])  # 6, 9 and (512 k each) 9 chunks, the last one a part
+@pytest.mark.parametrize("R, kblock", [(6, False), (16, True), (17, False), (32, False), (32, True)])
+def test_gate_up_bits(device, H, R, kblock):
+    print(f"case H {H} rows {R} kblock {kblock}", flush=True)
+    E, k, I, few = 32, 4, 1056, 64
+    g = torch.Generator().manual_seed(H + R)
+    half = torch.randn(E, H // 2, 2 * I, generator=g) * H ** -0.5
+    gu = torch.cat([half, -half + 2.0 ** -7 * torch.randn(E, H // 2, 2 * I, generator=g) * H ** -0.5], 1).to(BF)
+    first = torch.cat([gu[:, :, :few], gu[:, :, I:I + few]], 2)
+    x = torch.randn(R, H // 2, generator=g)
+    tx = torch.cat([x, x], 1).to(BF).reshape(1, 1, R, H).to(device.torch)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(R)]).to(torch.int16)
+    tid = ids.reshape(1, 1, R, k).to(device.torch)
+    tw = torch.softmax(torch.randn(1, 1, R, k, generator=g), -1).to(BF).to(device.torch)
+    u = len(set(ids.flatten().tolist()))
+
+    def h(w, n):
+        P = moe8.pack(device, w, torch.zeros(E, n, H, dtype=BF), kblock=kblock)
+        return moe8.gate_up_rows(tx, P, tid, tw, k, R, loaders=2).cpu().reshape(-1, min(E, R * k), n)[:R, :u]
+
+    same("the first columns", h(gu, I)[:, :, :few], h(first, few))
