@@ -2124,16 +2124,16 @@ __device__ __forceinline__ void xl_chunk_bfp8_b1(const Args& a, const uint8_t* c
 // bfloat4_b: a step is block k / 128; MFMA D takes k = 32 kq + 8 D + j of the step
 template <int PW, int D = 1>
 __device__ __forceinline__ void xl_chunk_bfp4(const Args& a, const uint8_t* const* cb, const uint8_t* const* eb, int k0,
-                                              int k1, int lane, f32x4 (&acc)[PW][2], uint4* xs) {
+                                              int k1, int lane, f32x4 (&acc)[PW][2], uint4* xs, uint32_t xbytes = 0) {
     static_assert(D == 1 || D == 2, "xl_chunk_bfp4: one or two steps in flight");
     const int ns = (k1 - k0) >> 7;
     if constexpr (D > 1) {
         if (ns % D) {
-            xl_chunk_bfp4<PW, 1>(a, cb, eb, k0, k1, lane, acc, xs);
+            xl_chunk_bfp4<PW, 1>(a, cb, eb, k0, k1, lane, acc, xs, xbytes);
             return;
         }
     }
-    const XStage<16> xst(a, lane);
+    const XStage<16> xst(a, lane, xbytes);
     uint4 cn[D][PW];
     uint32_t en[PW], e[PW];
     auto issue_x = [&](int s) { xst.stage(k0 + 128 * s, xs); };
@@ -2545,9 +2545,10 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
                 mgroup_bfp4<MT, PW>(b, cbx, ebx, gg, lane, acc);
         }
     };
-    // 32 rows of gate/up: x through each wavefront's LDS staging, as the dense 32-row kernel reads it (the same sums;
-    // x read in whole lines)
+    // 32 rows: x through each wavefront's LDS staging, as the dense 32-row kernel reads it (the same sums; x read in
+    // whole lines). The down's chunk views x from its unit's block on, so its staging may read only up to x's end.
     constexpr bool XLG = MOE == DR_MOE_GATE_UP_ROWS && MT == 2 && !KB;
+    constexpr bool XLD = MOE == DR_MOE_DOWN_ROWS && MT == 2 && !KB;
     uint4* xs = reinterpret_cast<uint4*>(part) + wave * (XS_BYTES / 16);
     const int ch1 = min((split + 1) * a.cps, a.chunks);
     const int nch = moe_n<MOE>() ? a.chains : a.waves;  // (the down modes: a chain a wavefront)
@@ -2574,7 +2575,12 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
                     cbe[q] = cb[q] + (size_t)e * a.cstride;
                     ebe[q] = eb[q] + (size_t)e * a.estride;
                 }
-                chunk(b, cbe, ebe, k0 - s * a.ekp, k1 - s * a.ekp);
+                if constexpr (XLD) {
+                    const uint32_t xb = 2u * (uint32_t)a.ldx * (uint32_t)a.m - 2u * (uint32_t)(s * a.ek);  // (to x's end)
+                    xl_chunk_bfp4<PW>(b, cbe, ebe, k0 - s * a.ekp, k1 - s * a.ekp, lane, acc, xs, xb);
+                } else {
+                    chunk(b, cbe, ebe, k0 - s * a.ekp, k1 - s * a.ekp);
+                }
             } else {
                 if constexpr (XLG)
                     xl_chunk_bfp4<PW>(a, cb, eb, k0, k1, lane, acc, xs);
@@ -2582,7 +2588,7 @@ __global__ __launch_bounds__(512) void dr_mfma_moe(const MoeArgs a) {
                     chunk(a, cb, eb, k0, k1);
             }
         }
-        if constexpr (XLG) __syncthreads();  // (every wavefront, one chain each, done with its staging before any
+        if constexpr (XLG || XLD) __syncthreads();  // (every wavefront, one chain each, done with its staging before any
                                              // partial lands on it)
 #pragma unroll
         for (int q = 0; q < PW; ++q)
@@ -3321,7 +3327,7 @@ template <int MT, int PW, int MOE>
 void launch_mfma_moe(const MoeArgs& a, int grid, hipStream_t st) {
     const dim3 b(64 * a.waves);
     size_t lds = (size_t)max(a.chains, a.splits) * PW * 16 * MT * 16 * sizeof(float);
-    if (MOE == DR_MOE_GATE_UP_ROWS && MT == 2)
+    if (MT == 2 && a.seg[0].fmt == DR_BFP4)
         lds = max(lds, (size_t)a.waves * XS_BYTES);  // (the x staging)
     if (a.seg[0].fmt == DR_BFP4_KB)
         hipLaunchKernelGGL((dr_mfma_moe<MT, PW, MOE, true>), dim3(grid), b, lds, st, a);
@@ -3368,13 +3374,12 @@ hipError_t launch_moe(const MoeArgs& a, int mode, int rows, int pw, int grid, hi
                         : launch_gemv_moe<2, 2, DR_MOE_DOWN_ROWS>(a, grid, st);
             else if (rows == 16)
                 launch_mfma_moe<1, 2, DR_MOE_DOWN_ROWS>(a, grid, st);
-            else if (a.seg[0].fmt == DR_BFP4) {
+            else if (a.pairs > 0) {
                 const size_t unit = 2 * 32 * 16 * sizeof(float);  // a tile's partial sums
                 const size_t lds = max((size_t)a.waves * XS_BYTES, (size_t)(a.waves + max(a.waves, a.splits)) * unit);
                 hipLaunchKernelGGL(dr_mfma_moe_down_pairs, dim3(a.pairs), dim3(64 * a.waves), lds, st, a);
             } else
-                hipLaunchKernelGGL((dr_mfma_moe<2, 2, DR_MOE_DOWN_ROWS, true>), dim3(grid), dim3(64 * a.waves),
-                                   (size_t)max(a.chains, a.splits) * 2 * 32 * 16 * sizeof(float), st, a);
+                launch_mfma_moe<2, 2, DR_MOE_DOWN_ROWS>(a, grid, st);
             break;
     }
     return hipGetLastError();
@@ -4058,6 +4063,31 @@ int dr_version(void) { return 1; }
 
 namespace {
 
+// dr_mfma_moe_down_pairs' K splits: as many as keep two workgroups on every CU in one round (45 pairs of the gpt-oss
+// shape in 11), each wavefront with a step at least
+int down_pair_splits(const MoeArgs& a, int units, int tiles) {
+    const int tp = (tiles + 1) / 2, most = units * ((a.ek + 127) / 128);
+    if (tiles > SPLIT_MAXTILES) return 1;
+    return std::max(1, std::min({2 * cu_count() / tp, DOWN_SPLITS, (most + MAXW - 1) / MAXW}));
+}
+
+// Whether the down of 17 to 32 rows takes less time in tile pairs than a tile a workgroup (a holds that plan). Both
+// times in us, as fitted to 356 shapes on MI355X (8 to 64 experts, H 256 to 4096, I 128 to 2880, 17 and 32 rows; within
+// 7 and 3 % of the measured ones at the mean): a workgroup's start and end, the splits' meeting, then the steps of 128 k
+// of its wavefronts, with one workgroup on a CU and with more. The pairs keep every CU busy for the whole of K at the
+// larger shapes (H = I = 2880, 32 experts: 91 -> 66 us), but cost more where a wavefront has few steps or their few
+// splits leave CUs idle (H = 1536, I = 768, 17 rows of top 1: 16.3 against 22.6; H = 512, I = 2048, 64 experts: 31 and
+// 46). A float32 y stays with the one-tile kernel, whose wavefronts sum at most 1024 k each. Over the 356, the choice is up to 4 % slower than the one-tile kernel alone and 5 % faster at the mean.
+bool down_in_pairs(const MoeArgs& a, double chosen, int tiles, int pair_splits) {
+    const double cus = cu_count(), steps = chosen * ((a.ek + 127) / 128);
+    const int per = (a.cps + MAXW - 1) / MAXW * a.kch / 128;  // a wavefront's steps
+    const double wgs = tiles * std::max(1., chosen * a.ekp / a.kch / a.cps);
+    const double one = 6.6 + 0.6 * a.splits + 1.9 * std::max(1., std::ceil(wgs / cus)) * per;
+    const double pairs = 7.8 + (pair_splits > 1 ? 3.5 : 0.) + 0.66 * pair_splits +
+                         steps / (MAXW * pair_splits) * (2.93 * std::ceil((tiles + 1) / 2 * pair_splits / cus) - 0.5);
+    return !a.y_f32 && pairs + 1. < one;
+}
+
 // the base launch's arguments (prepare), then the gather's: the tiles of the gate/up modes, the gathered K of the
 // down modes, the rows a pass
 int prepare_moe(const dr_launch* L, const dr_moe* M, MoeArgs& a, int& pw, int& tiles, int& mr) {
@@ -4131,15 +4161,16 @@ int prepare_moe(const dr_launch* L, const dr_moe* M, MoeArgs& a, int& pw, int& t
         a.ekp = ekp;
         a.seg[0].pstride = (unsigned)((ekp / kblk(DR_BFP4)) * 1024);
         if (ekp % a.kch) plan_chunks(a.k_pad, 256, &a.chunks, &a.kch, &a.waves, &a.splits, &a.cps);  // (a chunk in one unit)
-        // 32 rows of bfloat4_b: tile pairs, in as many splits as keep two workgroups on every CU in one round (45 pairs of
-        // the gpt-oss shape in 11), each wavefront a run of the union's 128-k steps of its own
+        // 32 rows of bfloat4_b in tile pairs where that takes less time
         if (mr == 32 && a.seg[0].fmt == DR_BFP4) {
-            const int tp = (a.seg[0].tiles + 1) / 2, most = units * ((a.ek + 127) / 128);
-            a.waves = MAXW;
-            a.splits = std::max(1, std::min({2 * cu_count() / tp, DOWN_SPLITS, (most + MAXW - 1) / MAXW}));
-            a.cps = (a.chunks + a.splits - 1) / a.splits;
-            if (tiles > SPLIT_MAXTILES) a.splits = 1;
-            a.pairs = tp * a.splits;
+            limit_splits(a);
+            const int pair_splits = down_pair_splits(a, units, tiles);
+            if (down_in_pairs(a, chosen, tiles, pair_splits)) {
+                a.waves = MAXW;
+                a.splits = pair_splits;
+                a.cps = (a.chunks + a.splits - 1) / a.splits;
+                a.pairs = (tiles + 1) / 2 * a.splits;
+            }
         }
         // The GEMV's tile width and K splits (the down modes have no block lists, so they may depend on N): the pair
         // of the lowest cost, ceil(workgroups / CUs) rounds of cps chunks x the width each plus a workgroup's fixed

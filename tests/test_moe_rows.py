@@ -1,7 +1,8 @@
-"""The MoE over 3 to 32 rows at the edges of its plans. test_down_rows: dr_mfma_moe_down_pairs (17 to 32 rows of
-bfloat4_b experts: tiles in pairs, the union's 128-k steps shared out over the splits' wavefronts), one tile and an odd
-count of tiles (H), an expert's K of a part of a step, of a step, of one more than a step and of many (I), unions of one
-expert (fewer steps than wavefronts) up to all of them, one split and several. Against the float64 sum over h as the
+"""The MoE over 3 to 32 rows at the edges of its plans. test_down_rows: the two kernels of the down of 17 to 32 rows of
+bfloat4_b experts, a tile a workgroup in chunks (one) and dr_mfma_moe_down_pairs (pairs: tiles in pairs, the union's 128-k
+steps shared out over the splits' wavefronts), each with one tile and an odd count of tiles (H), an expert's K of a part
+of a step, of a step, of a part more than steps and of many (I), unions of one expert (fewer steps than wavefronts) up to
+all of them, one split and several. The kernel that 256 CUs run each on stands beside it. Against the float64 sum over h as the
 device holds it, so the bound is derived: y is a bf16 rounding (2^-9 of the value) of float32 sums of exact products,
 whose order costs at most n 2^-24 of the sum of the products' magnitudes, n their count. test_gate_up_rows: the same
 bound carried through the activation."""
@@ -21,13 +22,17 @@ BF = torch.bfloat16
 
 # experts, slots, H, I, rows
 @pytest.mark.parametrize("E, k, H, I, R", [
-    (2, 1, 32, 32, 17),  # one tile, a part of a step an expert
-    (1, 1, 96, 128, 32),  # three tiles, one expert of one step
-    (4, 2, 64, 160, 24),  # a step and a part
-    (32, 4, 160, 480, 31),
-    (8, 8, 1056, 1408, 32),  # every expert chosen by every row; 33 tiles
-    (16, 2, 2080, 256, 18),  # 65 tiles in several splits
-    (4, 1, 17440, 96, 20),  # more tile pairs than two a CU: one split
+    (2, 1, 32, 32, 17),  # pairs: one tile, a part of a step an expert
+    (1, 1, 96, 128, 32),  # pairs: three tiles, one expert of one step
+    (4, 2, 64, 160, 24),  # one: a step and a part
+    (32, 4, 160, 480, 31),  # one: five tiles
+    (8, 8, 1056, 1408, 32),  # pairs: every expert chosen by every row; 33 tiles in 11 splits
+    (16, 2, 2080, 256, 18),  # one: 65 tiles in several splits
+    (4, 1, 17440, 96, 20),  # pairs: more of them than two a CU, one split
+    (16, 4, 4128, 288, 32),  # pairs: 129 tiles, two steps and a part, 6 splits
+    (16, 4, 4128, 288, 18),  # pairs: 4 experts chosen of the 16 expected
+    (4, 4, 8224, 160, 17),  # pairs: one split
+    (8, 4, 1024, 768, 32),  # one: every wavefront two chunks of 256 k
 ])
 def test_down_rows(device, E, k, H, I, R):
     print(f"case E {E} k {k} H {H} I {I} rows {R}", flush=True)
