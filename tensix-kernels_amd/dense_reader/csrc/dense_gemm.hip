@@ -409,8 +409,9 @@ __global__ __launch_bounds__(64 * GEMM_W, 1) void dr_gemm(const GemmArgs a) {
             for (int i = 0; i < 16; ++i) acc[n][t][i] = 0.f;
     gemm_k_loop<MT, FMT, GLU, KS>(a, nt, m0, acc, x0, x1, x2, x3);
     // The sums through LDS, an x stage for each wavefront, so that a store covers whole runs of a row: row r's 16-byte
-    // chunk k (columns 4 k .. + 3 of the two tiles) at 16 r + (k ^ (r % 16)).
-    __syncthreads();
+    // chunk k (columns 4 k .. + 3 of the two tiles) at 16 r + (k ^ (r % 16)). (The K loop ends with loads to the stages
+    // in flight, which must have landed, every wavefront's, before sums are written there.)
+    step_barrier<0, true>();
     constexpr int TP = KS ? MT : MT / 2;  // row tiles a pass
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 31, h = lane >> 5;

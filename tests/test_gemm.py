@@ -135,7 +135,9 @@ def test_columns_past_k_and_nan(device):
 def test_staging_order():
     """In the emitted gfx950 code of dr_gemm every barrier of the K loop follows a wait for the wavefront's LDS reads
     (lgkmcnt(0)) and for all but its newest x loads (vmcnt of at most two stages), and between two such barriers lie one
-    stage's loads to LDS, so that a stage is read only after its loads have landed and overwritten only after its reads."""
+    stage's loads to LDS, so that a stage is read only after its loads have landed and overwritten only after its reads.
+    After the loop's last loads every wavefront waits for all of its own (vmcnt(0)) at a barrier before the first sum is
+    written over a stage."""
     import __graft_entry__ as G
 
     hipcc = G.HIPCC if Path(G.HIPCC).exists() else shutil.which("hipcc")
@@ -163,5 +165,9 @@ def test_staging_order():
                 nxt = next(s for s in lines[a + 1:] if not s.startswith("s_waitcnt"))
                 assert nxt == "s_barrier", (name, lines[a], nxt)
             assert sum(a < i < b for i in dma) == stage, (name, a, b)
+        # all of the sums' 8 mt LDS writes (others are the ragged K's zeros)
+        end = [i for i in range(dma[-1], len(lines) - 1)
+               if re.match(r"s_waitcnt vmcnt\(0\) lgkmcnt\(0\)$", lines[i]) and lines[i + 1] == "s_barrier"]
+        assert end and sum(s.startswith("ds_write_b128") for s in lines[end[0]:]) >= 8 * mt, (name, end[:1])
         found += 1
     assert found == 30, found
