@@ -21,7 +21,7 @@ struct GemmArgs {
     SegDev seg;
 };
 
-// mt: row tiles of 32 a workgroup (2, 4, 6 or 8); ks: the wavefronts split K (mt 2)
+// mt: row tiles of 32 a workgroup (2, 4, 6 or 8; 2 for a float32 y); ks: the wavefronts split K (mt 2)
 hipError_t launch_gemm(const GemmArgs& g, int mt, bool ks, hipStream_t st);
 
 // LDS bytes a workgroup: four stages of x, 64 k of its rows each (ks: one for each wavefront)

@@ -85,7 +85,11 @@ struct StepCodes {
 // MT row tiles of 32, two column tiles of 32 a wavefront (with GLU the gate's and the up's). KS: the wavefronts split
 // K instead of lying side by side. acc: lane l's sums, row 32 t + l % 32, columns 8 g + 4 (l / 32) + 0 .. 3 of tile n in
 // words 4 g + 0 .. 3.
-template <int MT, int FMT, bool GLU, bool KS>
+// F32 (a float32 y, which shows the sums' rounding): the accumulators hold 256 k at a time, added up in three levels of
+// eight. One accumulator for all of K rounds at each of its K / 16 MFMAs, which at K = 4096 and 14336 was 2.5 and
+// 4.5 times the error of the passes of 32 rows (bfloat8_b 2.0e-7 against 8.0e-8, 4.7e-7 against 1.04e-7); so it is no
+// larger than theirs (7.4e-8, 8.7e-8; measured at K = 96 to 28672, each format).
+template <int MT, int FMT, bool GLU, bool KS, bool F32>
 __device__ __forceinline__ void gemm_k_loop(const GemmArgs& a, int nt, int m0, f32x16 (&acc)[2][MT], uint4* x0, uint4* x1,
                                             uint4* x2, uint4* x3) {
     constexpr int OT = GLU ? 1 : 2;                            // output tiles a wavefront
@@ -226,6 +230,13 @@ __device__ __forceinline__ void gemm_k_loop(const GemmArgs& a, int nt, int m0, f
         if constexpr (q == 3) B[n][u].w = w;
     };
 
+    f32x16 l1[2][F32 ? MT : 1], l2[2][F32 ? MT : 1], l3[2][F32 ? MT : 1];  // sums of 256, 2048 and 16384 k
+    if constexpr (F32) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) l1[n][t] = l2[n][t] = l3[n][t] = acc[n][t];  // (zeros)
+    }
     StepCodes<FMT> k0, k1, k2, k3;  // step s's codes in k[s % 4], asked for three steps ahead
     uint4 B0[2][4], B1[2][4];       // the decoded operands of even and odd steps (bf16 weights: the codes themselves)
     uint4 A[PF + 1];
@@ -303,6 +314,27 @@ __device__ __forceinline__ void gemm_k_loop(const GemmArgs& a, int nt, int m0, f
         step(4 * g + 1, ic<1>{}, x1, x2, x0, B1, B0, k1, k2, k0);
         step(4 * g + 2, ic<2>{}, x2, x3, x1, B0, B1, k2, k3, k1);
         step(4 * g + 3, ic<3>{}, x3, x0, x2, B1, B0, k3, k0, k2);
+        if constexpr (F32) {
+            auto carry = [](f32x16 (&to)[2][MT], f32x16 (&from)[2][MT]) {
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) {
+                        to[n][t] += from[n][t];
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) from[n][t][i] = 0.f;
+                    }
+            };
+            carry(l1, acc);
+            if (((g - g0) & 7) == 7) carry(l2, l1);
+            if (((g - g0) & 63) == 63) carry(l3, l2);
+        }
+    }
+    if constexpr (F32) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[n][t] = l3[n][t] + l2[n][t] + l1[n][t];
     }
 }
 
@@ -327,7 +359,7 @@ __device__ __forceinline__ ColScales col_scales(const SegDev& sd, int oc) {
 
 // 4 output columns oc .. oc + 3 (within the weight's) of row m, summed in g (and u): the scales, the GLU and the
 // residual, to y
-template <bool GLU>
+template <bool GLU, bool F32>
 __device__ __forceinline__ void gemm_store(const GemmArgs& a, int m, int oc, f32x4 g, f32x4 u, const ColScales& s) {
     const int left = a.seg.n_out - oc;
     const size_t ycol = (size_t)a.seg.col0 + oc;
@@ -344,7 +376,7 @@ __device__ __forceinline__ void gemm_store(const GemmArgs& a, int m, int oc, f32
         }
     }
     const size_t idx = (size_t)m * a.ldy + ycol;
-    if (a.y_f32) {
+    if constexpr (F32) {
         float* y = reinterpret_cast<float*>(a.y) + idx;
         if (a.vec4 && left >= 4) {
             *reinterpret_cast<f32x4*>(y) = f32x4{v[0], v[1], v[2], v[3]};
@@ -393,7 +425,7 @@ __device__ __forceinline__ void gemm_store_plain(const GemmArgs& a, uint16_t* y,
     *reinterpret_cast<uint2*>(y) = o;
 }
 
-template <int MT, int FMT, bool GLU, bool KS>
+template <int MT, int FMT, bool GLU, bool KS, bool F32>
 __global__ __launch_bounds__(64 * GEMM_W, 1) void dr_gemm(const GemmArgs a) {
     constexpr int BM = 32 * MT, OT = GLU ? 1 : 2;
     constexpr int XN = BM * 8 * (KS ? GEMM_W : 1);  // 16-byte chunks a stage of x
@@ -407,7 +439,7 @@ __global__ __launch_bounds__(64 * GEMM_W, 1) void dr_gemm(const GemmArgs a) {
         for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[n][t][i] = 0.f;
-    gemm_k_loop<MT, FMT, GLU, KS>(a, nt, m0, acc, x0, x1, x2, x3);
+    gemm_k_loop<MT, FMT, GLU, KS, F32>(a, nt, m0, acc, x0, x1, x2, x3);
     // The sums through LDS, an x stage for each wavefront, so that a store covers whole runs of a row: row r's 16-byte
     // chunk k (columns 4 k .. + 3 of the two tiles) at 16 r + (k ^ (r % 16)). (The K loop ends with loads to the stages
     // in flight, which must have landed, every wavefront's, before sums are written there.)
@@ -422,7 +454,7 @@ __global__ __launch_bounds__(64 * GEMM_W, 1) void dr_gemm(const GemmArgs a) {
     const ColScales cs = col_scales<GLU>(a.seg, oc);
     constexpr int RS = 64 / (8 * OT) * (KS ? GEMM_W : 1);  // rows a turn
     const int r0 = (KS ? (int)threadIdx.x : lane) / (8 * OT);
-    const bool plain = a.vec4 && !a.y_f32 && a.res == nullptr && a.seg.n_out - oc >= 4;
+    const bool plain = a.vec4 && !F32 && a.res == nullptr && a.seg.n_out - oc >= 4;
 #pragma unroll
     for (int tb = 0; tb < MT; tb += TP) {
         if (tb) __builtin_amdgcn_wave_barrier();
@@ -466,28 +498,28 @@ __global__ __launch_bounds__(64 * GEMM_W, 1) void dr_gemm(const GemmArgs a) {
             for (int row = r0; row < rows; row += RS) {
                 f32x4 g, u;
                 sums(row, g, u);
-                gemm_store<GLU>(a, m0 + 32 * tb + row, oc, g, u, cs);
+                gemm_store<GLU, F32>(a, m0 + 32 * tb + row, oc, g, u, cs);
             }
         }
     }
 }
 
-template <int MT, bool KS>
+template <int MT, bool KS, bool F32>
 void launch_gemm_t(const GemmArgs& g, hipStream_t st) {
     const dim3 grid(g.tm * g.tn), b(64 * GEMM_W);
     const bool glu = g.seg.glu != 0;
     switch (g.seg.fmt) {
         case DR_BFP8:
-            if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BFP8, true, KS>), grid, b, 0, st, g);
-            else hipLaunchKernelGGL((dr_gemm<MT, DR_BFP8, false, KS>), grid, b, 0, st, g);
+            if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BFP8, true, KS, F32>), grid, b, 0, st, g);
+            else hipLaunchKernelGGL((dr_gemm<MT, DR_BFP8, false, KS, F32>), grid, b, 0, st, g);
             break;
         case DR_BFP4:
-            if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BFP4, true, KS>), grid, b, 0, st, g);
-            else hipLaunchKernelGGL((dr_gemm<MT, DR_BFP4, false, KS>), grid, b, 0, st, g);
+            if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BFP4, true, KS, F32>), grid, b, 0, st, g);
+            else hipLaunchKernelGGL((dr_gemm<MT, DR_BFP4, false, KS, F32>), grid, b, 0, st, g);
             break;
         default:
-            if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BF16, true, KS>), grid, b, 0, st, g);
-            else hipLaunchKernelGGL((dr_gemm<MT, DR_BF16, false, KS>), grid, b, 0, st, g);
+            if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BF16, true, KS, F32>), grid, b, 0, st, g);
+            else hipLaunchKernelGGL((dr_gemm<MT, DR_BF16, false, KS, F32>), grid, b, 0, st, g);
             break;
     }
 }
@@ -495,11 +527,12 @@ void launch_gemm_t(const GemmArgs& g, hipStream_t st) {
 }  // namespace
 
 hipError_t launch_gemm(const GemmArgs& g, int mt, bool ks, hipStream_t st) {
-    if (ks) launch_gemm_t<2, true>(g, st);
-    else if (mt == 8) launch_gemm_t<8, false>(g, st);
-    else if (mt == 6) launch_gemm_t<6, false>(g, st);
-    else if (mt == 4) launch_gemm_t<4, false>(g, st);
-    else launch_gemm_t<2, false>(g, st);
+    if (g.y_f32) ks ? launch_gemm_t<2, true, true>(g, st) : launch_gemm_t<2, false, true>(g, st);
+    else if (ks) launch_gemm_t<2, true, false>(g, st);
+    else if (mt == 8) launch_gemm_t<8, false, false>(g, st);
+    else if (mt == 6) launch_gemm_t<6, false, false>(g, st);
+    else if (mt == 4) launch_gemm_t<4, false, false>(g, st);
+    else launch_gemm_t<2, false, false>(g, st);
     return hipGetLastError();
 }
 

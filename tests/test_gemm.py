@@ -118,6 +118,37 @@ def test_glu(device, fmt, m, k, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fmt", list(FMTS))
+@pytest.mark.parametrize("m, k, n", [(132, 512, 96), (160, 4096, 512), (132, 4096, 8192), (131, 2080, 9000), (192, 16896, 64)])
+def test_float32_error(device, fmt, m, k, n):
+    """A float32 y is as exact as that of 32 rows a call, whose kernel sums K over eight wavefronts: its error against
+    float64 at most that of the same rows in calls of 32 (and a twentieth: 2 % is what another draw of the inputs moves
+    either)."""
+    tw, h = _weight(device, n, k, fmt, 41)
+    x, tx = _x(device, m, k, 42)
+    want = (x.to(torch.bfloat16).to(device.torch).double() @ h.to(device.torch).double()).cpu()
+    y = linear.matmul(tx, tw, None, out32=True).cpu().double().reshape(m, n)
+    parts = [linear.matmul(tx[..., r:r + 32, :].contiguous(), tw, None, out32=True).reshape(-1, n) for r in range(0, m, 32)]
+    one = torch.cat(parts).cpu().double()
+    err, ref = ((v - want).norm() / want.norm() for v in (y, one))
+    print(f"{fmt} rows {m} K {k} N {n}: {float(err):.3e}, in calls of 32 rows {float(ref):.3e}", flush=True)
+    assert err <= 1.05 * ref
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", list(FMTS))
+@pytest.mark.parametrize("m, k, n", [(65, 1056, 96), (200, 2336, 14400)])
+def test_glu_float32(device, fmt, m, k, n):
+    gw, uw = O.matrix(n, k, 51), O.matrix(n, k, 52)
+    hg, hu = (torch.from_numpy(O.held(w.T.contiguous(), fmt)).double().to(device.torch) for w in (gw, uw))
+    tg, tu = (linear.native_weight(device, w, FMTS[fmt])[0] for w in (gw, uw))
+    x, tx = _x(device, m, k, 53)
+    xd = x.to(torch.bfloat16).double().to(device.torch)
+    y = _host(linear.matmul(tx, tg, None, glu=True, w_up=tu, out32=True), m)
+    check(f"{fmt} swiglu float32", y, O.glu_ref((xd @ hg).cpu(), (xd @ hu).cpu(), "swiglu"), rel=1e-5, pcc=0.999999)
+
+
+@pytest.mark.gpu
 def test_columns_past_k_and_nan(device):
     """A ragged K: what lies past K in x's memory (the next row, here Inf and NaN) enters no sum; a NaN row stays its
     own row's."""
@@ -149,7 +180,7 @@ def test_staging_order():
     assert r.returncode == 0, r.stderr[-2000:]
     found = 0
     for name, body in re.findall(r"^(_ZN3drk\S*dr_gemmI\S*):(.*?)s_endpgm", r.stdout, re.M | re.S):
-        mt, ks = (int(v) for v in re.search(r"dr_gemmILi(\d+)ELi\dELb\dELb(\d)E", name).groups())
+        mt, ks = (int(v) for v in re.search(r"dr_gemmILi(\d+)ELi\dELb\dELb(\d)ELb\dE", name).groups())
         stage = 4 * mt if ks else mt  # loads to LDS a stage, of one wavefront
         lines = [s.strip() for s in body.split("\n")]
         lines = [s for s in lines if s and not s.startswith((";", ".")) and not s.endswith(":")]
@@ -162,7 +193,7 @@ def test_staging_order():
         assert [v for _, v in waits if v != stage] == [2 * stage] and sum(i < inside[0] for i in dma) == 3 * stage
         for a, b in zip(inside, inside[1:] + [len(lines)]):
             if not ks:
-                nxt = next(s for s in lines[a + 1:] if not s.startswith("s_waitcnt"))
+                nxt = next(s for s in lines[a + 1:] if s == "s_barrier" or s.startswith(("ds_", "buffer_", "global_", "flat_")))
                 assert nxt == "s_barrier", (name, lines[a], nxt)
             assert sum(a < i < b for i in dma) == stage, (name, a, b)
         # all of the sums' 8 mt LDS writes (others are the ragged K's zeros)
@@ -170,4 +201,4 @@ def test_staging_order():
                if re.match(r"s_waitcnt vmcnt\(0\) lgkmcnt\(0\)$", lines[i]) and lines[i + 1] == "s_barrier"]
         assert end and sum(s.startswith("ds_write_b128") for s in lines[end[0]:]) >= 8 * mt, (name, end[:1])
         found += 1
-    assert found == 30, found
+    assert found == 42, found
