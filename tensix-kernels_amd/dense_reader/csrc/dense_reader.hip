@@ -3716,8 +3716,24 @@ constexpr GemmTile GEMM_TILES[] = {{2, true, 100, 28}, {2, false, 300, 66}, {4, 
 // a float32 y: a round of ks 9, 21 and 66 us at K = 1024, 4096 and 14336, of 64 rows 21, 65 and 193 (dense_gemm.hip's F32)
 constexpr GemmTile GEMM_TILES_F32[] = {{2, true, 400, 28}, {2, false, 700, 80}};
 
-// false: the launch runs in passes
-bool gemm_plan(const dr_launch* L, const Args& a, GemmArgs& g, GemmTile& best) {
+// The passes' time in the same unit: each pass a start and end, the splits' meeting and, for each round of workgroups
+// over the CUs, a wavefront's k (1024 of them 12.6 us, bf16's 16; of a GLU's two weights 13 and 22). A last pass of at
+// most 16 of 32 rows takes three quarters of one.
+long long passes_cost(const Args& a) {
+    const bool glu = a.seg[0].glu != 0, bf16 = a.seg[0].fmt == DR_BF16;
+    const int wk = (a.cps + a.waves - 1) / a.waves * a.kch, b = glu ? (bf16 ? 2200 : 1300) : (bf16 ? 1600 : 1260);
+    const int last = a.m % 32;
+    const long long quarters = glu ? 4 * ((a.m + 15) / 16) : 4 * (a.m / 32) + (last == 0 ? 0 : last <= 16 ? 3 : 4);
+    const long long rounds = ((long long)a.tiles * a.splits + cu_count() - 1) / cu_count();
+    return quarters * (440 + 80 * a.splits + rounds * wk * b / 1024) / 4;
+}
+
+// false: the launch runs in passes. For a long K (past 14336, or 4096 with a float32 y) that is where they take less time than the tiles (whose times above
+// are up to a fifth too long, a float32 y's apart): few tiles of a long K leave most CUs without a workgroup of dr_gemm,
+// while the passes split K over workgroups (GLU of 33 rows K = 28672 N = 512 bfloat8_b 110 us, 61 in passes; 129 rows
+// K = 57344 N = 32 209 and 97). Over 1704 calls of K = 512 to 57344 the choice is within 0.1 % of the better one at the
+// mean, and up to 11 % slower than the passes alone (8 calls by more than 4 %, K = 18432 and more). Passes that need more workspace than dr_matmul_noalloc has are not an option.
+bool gemm_plan(const dr_launch* L, const Args& a, int pw, int mr, GemmArgs& g, GemmTile& best) {
     if (L->m < (a.seg[0].glu ? GEMM_MIN_M_GLU : GEMM_MIN_M) || a.nseg != 1 || a.rec != nullptr || a.seg[0].fmt > DR_BF16) return false;
     const SegDev& s = a.seg[0];
     g = GemmArgs{};
@@ -3751,7 +3767,8 @@ bool gemm_plan(const dr_launch* L, const Args& a, GemmArgs& g, GemmTile& best) {
         g.tn = (int)tn;
     }
     // (a tile's rows of x lie within the buffer loads' 31-bit offsets)
-    return least >= 0 && (int64_t)a.ldx * 2 * 256 < INT32_MAX;
+    if (least < 0 || (int64_t)a.ldx * 2 * 256 >= INT32_MAX) return false;
+    return 5 * passes_cost(a) >= (a.y_f32 ? 5 : 4) * least || workspace_bytes(a, pw, mr) > DR_SCRATCH_BYTES;
 }
 
 // dr_matmul's launches: one pass of up to mr rows each (the passes a top-k launch needs, not y, skipped)
@@ -3867,7 +3884,7 @@ int64_t dr_workspace_bytes(const dr_launch* L) {
     if (prepare(L, a, pw, tiles, mr) != DR_OK) return -1;
     GemmArgs g;
     GemmTile gt;
-    if (gemm_plan(L, a, g, gt)) return 0;
+    if (gemm_plan(L, a, pw, mr, g, gt)) return 0;
     return workspace_bytes(a, pw, mr);
 }
 
@@ -3879,7 +3896,7 @@ int dr_matmul(const dr_launch* L) {
     if (st0 != DR_OK) return st0;
     GemmArgs g;
     GemmTile gt;
-    if (gemm_plan(L, a, g, gt)) return hip_status(launch_gemm(g, gt.mt, gt.ks, S(L->stream)));
+    if (gemm_plan(L, a, pw, mr, g, gt)) return hip_status(launch_gemm(g, gt.mt, gt.ks, S(L->stream)));
     const int64_t need = workspace_bytes(a, pw, mr);
     if (need > 0) {
         // split K needs the workspace: its counters start at zero (the caller zeroes it once; each launch leaves
@@ -3909,7 +3926,7 @@ int dr_matmul_noalloc(const dr_launch* L) {
     if (st0 != DR_OK) return st0;
     GemmArgs g;
     GemmTile gt;
-    if (gemm_plan(L, a, g, gt)) return hip_status(launch_gemm(g, gt.mt, gt.ks, S(L->stream)));
+    if (gemm_plan(L, a, pw, mr, g, gt)) return hip_status(launch_gemm(g, gt.mt, gt.ks, S(L->stream)));
     const int64_t need = workspace_bytes(a, pw, mr);
     if (need > DR_SCRATCH_BYTES) return DR_ERANGE;  // (checked before any device call)
     hipStream_t st = S(L->stream);
@@ -3932,7 +3949,7 @@ int dr_launch_plan(const dr_launch* L, dr_launch_info* info) {
     *info = dr_launch_info{};
     GemmArgs g;
     GemmTile gt;
-    if (gemm_plan(L, a, g, gt)) {
+    if (gemm_plan(L, a, pw, mr, g, gt)) {
         info->kernel = 1;
         info->rows_per_pass = 32 * gt.mt;
         info->tile_cols = TILE;
@@ -3984,7 +4001,7 @@ int dr_launch_work(const dr_launch* L, int32_t* work, int max_workgroups) {
     if (st != DR_OK) return st;
     GemmArgs gm;
     GemmTile gt;
-    if (gemm_plan(L, a, gm, gt)) {  // (a row tile's workgroups, one a column tile)
+    if (gemm_plan(L, a, pw, mr, gm, gt)) {  // (a row tile's workgroups, one a column tile)
         if (gm.tn > max_workgroups) return DR_ERANGE;
         const int per = (a.seg[0].glu ? 1 : 2) * (gt.ks ? 1 : GEMM_W);
         for (int i = 0; i < gm.tn; ++i) {

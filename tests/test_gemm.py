@@ -15,7 +15,7 @@ import pytest
 import torch
 
 from common.testing import check, same
-from dense_reader import linear
+from dense_reader import _lib, linear
 from oracle import dense_oracle as O
 
 FMTS = {"bfp8": linear.bfloat8_b, "bfp4": linear.bfloat4_b, "bf16": linear.bfloat16}
@@ -33,6 +33,38 @@ def _weight(dev, n, k, fmt, seed):
 
 def _host(y, m):
     return y.float().cpu().reshape(m, -1)
+
+
+def test_passes_where_faster():
+    """On the host, for 256 CUs: up to K = 14336 (a float32 y: 4096) every call past the row limits is one tiled launch; for
+    a longer K the passes of 16 (GLU) and 32 rows stay where few tiles leave most CUs idle, unless their workspace would not fit
+    dr_matmul_noalloc's own."""
+    def plan(fmt, m, k, n, glu=False, f32=False):
+        L = _lib.Launch()  # device pointers that are never read: the plan only reads the launch's sizes
+        L.x, L.y, L.m, L.k, L.ldx, L.ldy, L.nseg, L.y_f32 = 16, 16, m, k, k, n, 1, int(f32)
+        s = L.seg[0]
+        s.fmt, s.n, s.n_pad, s.codes, s.exps = fmt, n, -(-n // 32) * 32, 16, 16
+        if glu:
+            s.glu, s.codes_up, s.exps_up = 2, 16, 16
+        return _lib.launch_info(L), _lib.lib().dr_workspace_bytes(L)
+
+    for fmt in (0, 1, 2):
+        for f32 in (False, True):
+            for k in (96, 1024, 4096, 14336)[:3 if f32 else 4]:
+                for n in (32, 512, 4096):
+                    for m, glu in ((33, True), (64, True), (129, False), (256, False)):
+                        p, need = plan(fmt, m, k, n, glu, f32)
+                        assert p["rows_per_pass"] >= 64 and need == 0, (fmt, m, k, n, glu, f32, p)
+            for m, glu, rows in ((33, True, 16), (129, False, 32)):
+                for k, n in ((28672, 512), (57344, 32)) if glu or fmt != 2 else ((57344, 32),):
+                    p, need = plan(fmt, m, k, n, glu, f32)
+                    assert (p["rows_per_pass"], p["splits"]) == (rows, -(-k // 8192)) and need > 0, (fmt, m, k, n, p)
+                p, need = plan(fmt, m, 28672, 14336, glu, f32)
+                assert p["rows_per_pass"] >= 64 and need == 0, (fmt, m, p)
+    cap = _lib.lib().dr_scratch_bytes()
+    for n in (32, 256, 512, 1024):
+        p, need = plan(0, 129, 1 << 20, n)
+        assert need <= cap and (p["rows_per_pass"] == 32) == (need > 0), (n, p, need)
 
 
 # (rows, K, N, rows a tile, output tiles a workgroup): every tile of the plan; rows past the last tile, K off the
