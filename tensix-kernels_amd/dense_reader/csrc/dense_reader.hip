@@ -2955,9 +2955,9 @@ __global__ __launch_bounds__(256) void dr_pack_kb_k(const float* __restrict__ w,
         make_uint2(word[0], word[1]);
 }
 
-// the values of a lane's 16 bytes (block b of its 256-k group) in k order
-template <int FMT, int I = 0, typename F>
-__device__ __forceinline__ void unpack_row(const uint32_t (&w)[4], uint32_t e, int b, F put) {
+// the values of a lane's 16 bytes (block b of its 256-k group) in k order, to out
+template <int FMT, int I = 0>
+__device__ __forceinline__ void unpack_row(const uint32_t (&w)[4], uint32_t e, int b, float* out) {
     constexpr int PER = kblk(FMT) / 4;
     if constexpr (I < PER) {
         float v;
@@ -2978,44 +2978,47 @@ __device__ __forceinline__ void unpack_row(const uint32_t (&w)[4], uint32_t e, i
             }
             v = __builtin_ldexpf((float)m, (int)(ev & 0xFFu) - 129);
         }
-        put(I, v);
-        unpack_row<FMT, I + 1>(w, e, b, put);
+        out[I] = v;
+        unpack_row<FMT, I + 1>(w, e, b, out);
     }
 }
 
-// A wavefront writes 64 columns (four panels, a column a lane) over 256 k of out: a lane's 16-byte loads hold
-// consecutive k of its column, each value's row of 64 columns is one 256-byte store, and the panel's exponents, a dword
-// a lane, are broadcast across the 16 lanes of the panel. (One thread a value, with its 64-bit divisions and byte loads,
-// took 152 us for bfloat8_b K = 4096 N = 14336; 75 us now, 4.0 TB/s.)
+// A wavefront writes 64 columns (four panels, a column a lane) over a quarter of a k-block: a lane's one 16-byte load
+// holds consecutive k of its column, each value's row of 64 columns is one 256-byte store, and the panel's exponents, a
+// dword a lane, are broadcast across the 16 lanes of the panel. So little a wavefront, because a small weight has few of
+// them and then takes as long as one: over 256 k each, K = 512 N = 512 bfloat8_b took 18.5 us, 2.6 so (and K = 4096
+// N = 14336 82 us, 54 so: 5.5 TB/s of codes and float values).
 template <int FMT>
 __global__ __launch_bounds__(256) void dr_unpack_k(const uint8_t* __restrict__ codes, const uint8_t* __restrict__ exps,
                                                    int n, int k, int n_pad, int k_pad, float* __restrict__ out,
                                                    long long ld_out) {
-    constexpr int KB = kblk(FMT), PER = KB / 4;  // k of a block, of a lane's load
+    constexpr int KB = kblk(FMT), PER = KB / 4, NB = 256 / KB;  // k of a block, of a lane's load; blocks of 256 k
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15;
     const int groups = (k + 255) / 256;
-    const long long item = (long long)blockIdx.x * 4 + wave;
+    const long long part = (long long)blockIdx.x * 4 + wave, item = part / (4 * NB);
     if (item >= (long long)((n + 63) / 64) * groups) return;
-    const int n0 = (int)(item / groups) * 64, g = (int)(item % groups);
-    const int p = min((n0 + lane) >> 4, n_pad / 16 - 1), col = n0 + lane;
-    const uint8_t* pc = codes + (size_t)p * (k_pad / KB) * 1024 + (size_t)(g * (256 / KB)) * 1024 + c * 16;
+    const int n0 = (int)(item / groups) * 64, g = (int)(item % groups), u = (int)(part % (4 * NB)), kq = u / NB, b = u % NB;
+    const int p = min((n0 + lane) >> 4, n_pad / 16 - 1), col = n0 + lane, kk = g * 256 + b * KB + kq * PER;
+    if (kk >= k) return;
+    const uint8_t* pc = codes + (size_t)p * (k_pad / KB) * 1024 + (size_t)(g * NB + b) * 1024 + (kq * 16 + c) * 16;
     const uint8_t* pe = FMT == DR_BF16 ? nullptr : exps + (size_t)p * k_pad + g * 256;
-    for (int kq = 0; kq < 4; ++kq) {
-        // bfp8 / bfp4: this lane's exponents (its k of each block, or its pair of k); kblock: the lane's column's own
-        uint32_t e = 0;
-        if (FMT == DR_BFP8 || FMT == DR_BFP4) e = *reinterpret_cast<const uint32_t*>(pe + 4 * (16 * kq + c));
+    // bfp8 / bfp4: this lane's exponents (its k of each block, or its pair of k); kblock: the lane's column's own
+    uint32_t e = 0;
+    if (FMT == DR_BFP8 || FMT == DR_BFP4) e = *reinterpret_cast<const uint32_t*>(pe + 4 * (16 * kq + c));
+    if (FMT == DR_BFP4_KB) e = *reinterpret_cast<const uint16_t*>(pe + b * 128 + (kq * 16 + c) * 2);
+    const uint4 q = *reinterpret_cast<const uint4*>(pc);
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+    float v[PER];
+    unpack_row<FMT>(w, e, b, v);
+    if (col >= n) return;
+    float* o = out + (long long)kk * ld_out + col;
+    if (kk + PER <= k) {
 #pragma unroll
-        for (int b = 0; b < 256 / KB; ++b) {
-            const uint4 q = *reinterpret_cast<const uint4*>(pc + b * 1024 + kq * 256);
-            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-            if (FMT == DR_BFP4_KB) e = *reinterpret_cast<const uint16_t*>(pe + b * 128 + (kq * 16 + c) * 2);
-            const int kk = g * 256 + b * KB + kq * PER;
-            float* o = out + (long long)kk * ld_out + col;
-            auto put = [&](int i, float v) {
-                if (kk + i < k && col < n) o[(long long)i * ld_out] = v;
-            };
-            unpack_row<FMT>(w, e, b, put);
-        }
+        for (int i = 0; i < PER; ++i) o[(long long)i * ld_out] = v[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (kk + i < k) o[(long long)i * ld_out] = v[i];
     }
 }
 
@@ -3482,7 +3485,7 @@ int dr_unpack(const void* codes, const void* exps, int fmt, int n, int k, int n_
         n_pad % 32 || ld_out < n || (fmt != DR_BF16 && exps == nullptr) || fmt < 0 || fmt > DR_BFP4_KB || fmt == DR_INT4)
         return DR_EINVAL;
     const long long items = (long long)((n + 63) / 64) * ((k + 255) / 256);
-    const unsigned grid = (unsigned)((items + 3) / 4);
+    const unsigned grid = (unsigned)(items * (256 / kblk(fmt)));  // (four wavefronts each: the quarters of a k-block)
     auto* c8 = reinterpret_cast<const uint8_t*>(codes);
     auto* e8 = reinterpret_cast<const uint8_t*>(exps);
     if (fmt == DR_BFP8)
