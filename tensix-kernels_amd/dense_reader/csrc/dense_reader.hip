@@ -3203,12 +3203,23 @@ int rows_per_pass(int m) {
     return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : 8;
 }
 
-// int4's rows a pass: the GEMV up to 5 rows (whose rows equal the one-token call's bit for bit), four a pass from 3 on,
-// then the MFMA kernel.
+// int4's rows a pass: the GEMV up to 5 rows, whose rows equal the one-token call's bit for bit (and are tested to), then
+// the MFMA kernel (K = 4096 N = 14336: 5 rows 21 us, 6 rows 13). Of 3 to 5 rows the GEMV takes four a pass where that is
+// faster than two: with a 32-column workgroup on every CU (3 rows K = 4096 N = 8192 and 14336 12.7 -> 9.7, 18.1 -> 13.9
+// us; below that two passes of short workgroups are, N = 4096 7.8 against 9.1, K = 8192 N = 32 10.4 against 13.8), and at
+// K of 512 and 1024 (5.1 -> 4.6 us); but not where a short K leaves many workgroups with little but their ends (K = 96
+// N = 65536 8.2 against 11.1). Both give the same bits.
 #ifndef DR_INT4_MFMA_M
 #define DR_INT4_MFMA_M 6
 #endif
-int int4_rows(int m) { return m >= DR_INT4_MFMA_M ? (m <= 16 ? 16 : 32) : m <= 2 ? m : 4; }
+int int4_rows(int m, int k, int tiles) {
+    if (m >= DR_INT4_MFMA_M) return m <= 16 ? 16 : 32;
+    if (m <= 2) return m;
+    int chunks, kch, waves, splits, cps;
+    plan(k, false, &chunks, &kch, &waves, &splits, &cps);
+    const bool full = (long long)tiles * splits >= cu_count();
+    return full ? (chunks >= 4 || tiles <= 4 * cu_count() ? 4 : 2) : (chunks >= 2 && chunks <= 4 ? 4 : 2);
+}
 
 // Set by dr_launch_plan while it walks the launch path: the dense launches then store their kernel's LDS bytes (static
 // plus dynamic) here instead of launching it.
@@ -3612,7 +3623,7 @@ int prepare(const dr_launch* L, Args& a, int& pw, int& tiles, int& mr, bool gath
     if (pw == 4 && mr == 32) mr = 16;  // and the LDS)
     if (a.seg[0].fmt == DR_INT4) {
         // (fewer rows a pass where their split-K sums would not fit the library's own workspace)
-        mr = int4_rows(L->m);
+        mr = int4_rows(L->m, L->k, tiles);
         const int narrower[] = {16, 4, 2};
         for (const int r : narrower) {
             plan(L->k, mr >= 16, &a.chunks, &a.kch, &a.waves, &a.splits, &a.cps);

@@ -20,13 +20,18 @@ def _plan(m, k, n):
 
 
 def test_plan_on_the_host():
-    """The kernel and rows a pass by rows; never tile pairs (those kernels read block-float weights only); and fewer rows
-    a pass where the split-K sums of a long K would not fit dr_matmul_noalloc's own workspace."""
+    """The kernel and rows a pass by rows; never tile pairs (those kernels read block-float weights only); 3 to 5 rows four
+    a pass or two by the workgroups and K; and fewer rows a pass where the split-K sums of a long K would not fit
+    dr_matmul_noalloc's own workspace."""
     for n in (78, 2048, 14336, 131072):
-        for m, kernel, rows in ((1, "gemv", 1), (2, "gemv", 2), (3, "gemv", 4), (5, "gemv", 4), (6, "mfma", 16),
+        few = 4 if n > 8000 else 2
+        for m, kernel, rows in ((1, "gemv", 1), (2, "gemv", 2), (3, "gemv", few), (5, "gemv", few), (6, "mfma", 16),
                                 (16, "mfma", 16), (17, "mfma", 32), (300, "mfma", 32)):
             p, _ = _plan(m, 4096, n)
             assert (p["kernel"], p["rows_per_pass"], p["tiles_per_workgroup"]) == (kernel, rows, 1), (m, n, p)
+    for k, n, rows in ((96, 32, 2), (96, 14336, 4), (96, 65536, 2), (512, 32, 4), (512, 65536, 2), (1024, 32, 4),
+                       (1024, 65536, 4), (2048, 4096, 2), (8192, 4096, 2), (14336, 4096, 4), (28672, 2048, 4)):
+        assert _plan(4, k, n)[0]["rows_per_pass"] == rows, (k, n)
     cap = _lib.lib().dr_scratch_bytes()
     for n, rows in ((14336, 32), (32768, 16), (65536, 4), (262144, 2)):
         p, need = _plan(32, 14336, n)
