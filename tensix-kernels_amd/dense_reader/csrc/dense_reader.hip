@@ -2313,8 +2313,9 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 template <int MT, int PW, int FMT, bool ONE>
-__global__ __launch_bounds__(512, MT == 2 ? 4 : 1) void dr_mfma(const Args a) {  // (32 rows: 4 wavefronts a SIMD, so
-                                                                                 // two workgroups a CU)
+// (32 rows: 4 wavefronts a SIMD, so two workgroups a CU; int4, which holds its x in registers, 2: at 128 registers its K
+// loop spilled 35 of them, K = 4096 N = 14336 17 and 32 rows 28, 33 us, 20 and 23 at 163)
+__global__ __launch_bounds__(512, MT == 2 ? (FMT == DR_INT4 ? 2 : 4) : 1) void dr_mfma(const Args a) {
     constexpr int ROWS = 16 * MT;
     extern __shared__ float part[];  // [W][PW][ROWS][16]
     __shared__ float tval[ROWS][TILE];

@@ -192,3 +192,34 @@ def test_split_k_meeting_order(library_asm):
     assert len(met) >= 20, f"only {len(met)} kernels with the meeting found: the scanner is not looking at them"
     bad = meeting_order_faults(asm)
     assert not bad, f"{len(bad)} kernels break the split-K handoff's order, e.g. {bad[:3]}"
+
+
+def scratch_in_mfma_loops(asm):
+    """[(function, scratch instructions)] of the innermost loops that hold both a matrix instruction and an access to
+    scratch memory: registers spilled inside a K loop."""
+    found = []
+    for name, body in re.findall(r"^(_Z\S+):(.*?)^\.Lfunc_end", asm, re.M | re.S):
+        lines = [s.split(";")[0].strip() for s in body.split("\n")]
+        at = {s[:-1]: i for i, s in enumerate(lines) if s.startswith(".LBB") and s.endswith(":")}
+        loops = [(at[t], i) for i, s in enumerate(lines) if s.startswith(("s_branch", "s_cbranch"))
+                 for t in [s.split()[1]] if at.get(t, i) < i]
+        for b, e in loops:
+            if any((b, e) != (b2, e2) and b <= b2 and e2 <= e for b2, e2 in loops):
+                continue
+            n = sum(s.startswith("scratch_") for s in lines[b:e])
+            if n and any(s.startswith("v_mfma") for s in lines[b:e]):
+                found.append((name, n))
+    return found
+
+
+def test_scratch_scanner_finds_a_planted_spill():
+    loop = "_Zk:\n.LBB0_1:\n\tv_mfma_f32_16x16x32_bf16 v[0:3], v[4:7], v[8:11], v[0:3]\n%s\ts_cbranch_scc1 .LBB0_1\n%s.Lfunc_end0:\n"
+    spill = "\tscratch_load_dword v9, off, off\n"
+    assert scratch_in_mfma_loops(loop % (spill, ""))
+    assert not scratch_in_mfma_loops(loop % ("", spill))
+
+
+def test_no_spill_in_a_k_loop(library_asm):
+    for name, asm in library_asm.items():
+        assert not scratch_in_mfma_loops(asm), (name, scratch_in_mfma_loops(asm))
+    assert any("v_mfma" in asm for asm in library_asm.values())
