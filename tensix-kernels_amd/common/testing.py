@@ -1,7 +1,7 @@
 """The test bars of the reference (common/testing.py:16-41 of XylolabsInc/tensix-kernels), for torch tensors.
 
 check: relative Frobenius error below rel and PCC above pcc, every value finite. same: bit for bit. raises: the
-exception type. Each prints one `ok` / `FAIL` line in the reference's format.
+exception type. within (not one of the reference's): every value within a bound of its own. Each prints one `ok` / `FAIL` line in the reference's format.
 """
 
 import torch
@@ -26,6 +26,14 @@ def same(name, a, b):
     ok = a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
     print(f"{'ok  ' if ok else 'FAIL'} {name}: bit for bit {'equal' if ok else 'DIFFERENT'}", flush=True)
     assert ok, name
+
+
+def within(name, y, r, bound):
+    """|y - r| at most bound at every value (r and bound float64, on y's device or the host)."""
+    y = y.detach().to(r.device).double()
+    over = ((y - r).abs() / bound).max().item() if bool(torch.isfinite(y).all()) else float("inf")
+    print(f"{'ok  ' if over <= 1 else 'FAIL'} {name}: worst {over:.4f} of its bound", flush=True)
+    assert over <= 1, (name, over)
 
 
 def raises(name, exc, fn):

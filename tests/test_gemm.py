@@ -2,10 +2,14 @@
 CPU oracle; and the order of its staging in the emitted code.
 
 Bars as for the other kernels (the reference's): 1 % relative Frobenius error and PCC 0.9999 for bf16 outputs, 0.1 % for
-fp32 outputs. Every row is its own MFMA column, summed in an order that depends on K and the tile only, so permuting x's
+fp32 outputs; and every value within a bound of its own against the products in float64 (a whole matrix's error hides a
+wrong column or store at an edge): the output's rounding, 2^-8 of the value (bf16) or 2^-23, and float32 sums of exact
+products in any order, at most K 2^-24 of the sum of their magnitudes (the scales, the GLU and the residual carried
+through). Every row is its own MFMA column, summed in an order that depends on K and the tile only, so permuting x's
 rows permutes y's bit for bit and repeated calls agree.
 """
 
+import math
 import re
 import shutil
 import subprocess
@@ -14,7 +18,7 @@ from pathlib import Path
 import pytest
 import torch
 
-from common.testing import check, same
+from common.testing import check, same, within
 from dense_reader import _lib, linear
 from oracle import dense_oracle as O
 
@@ -33,6 +37,28 @@ def _weight(dev, n, k, fmt, seed):
 
 def _host(y, m):
     return y.float().cpu().reshape(m, -1)
+
+
+def _products(tx, h):
+    """x @ h and its terms' magnitudes summed, in float64 on the GPU, and the latter's share of the sums' error."""
+    xd, hd = tx.double().reshape(-1, tx.shape[-1]), h.to(tx.device).double()
+    return xd @ hd, (xd.abs() @ hd.abs()) * (xd.shape[1] * 2.0**-24)
+
+
+def _glu(g, ge, u, ue, act):
+    """act(g) * u in float64 and its bound for errors of ge and ue (the activations' slopes are below 1.13 and their
+    float32 evaluation within 2^-18 of the argument)."""
+    z = 2 * (2 / math.pi) ** 0.5 * (g + 0.044715 * g**3) if act == "geglu" else g
+    a = g * torch.sigmoid(z)
+    ae = 1.13 * ge + g.abs() * 2.0**-18
+    return a * u, ae * u.abs() + a.abs() * ue + ae * ue
+
+
+ROUND = {torch.bfloat16: 2.0**-8, torch.float32: 2.0**-23}
+
+
+def _near(name, y, want, err):
+    within(name, y.reshape(want.shape), want, want.abs() * ROUND[y.dtype] + err + 1e-30)
 
 
 def test_passes_where_faster():
@@ -93,8 +119,12 @@ def test_tiles(device, fmt, m, k, n, rows, tiles):
     assert p["passes"] == -(-m // rows) and p["workgroups"] == -(-p["tiles"] // tiles)
     s = torch.rand(n, generator=torch.Generator().manual_seed(3)) + 0.5
     ts = linear.scale_tensor(device, s, dtype=linear.float32)
-    y = _host(linear.matmul(tx, tw, ts), m)
+    yd = linear.matmul(tx, tw, ts)
+    y = _host(yd, m)
     check(f"{fmt} rows {m} K {k} N {n} scaled", y, O.ref(x, h, s))
+    want, err = _products(tx, h)
+    sd = s.to(tx.device).double()
+    _near("every value", yd, want * sd, err * sd)
     same("repeated call", _host(linear.matmul(tx, tw, ts), m), y)
     perm = torch.randperm(m, generator=torch.Generator().manual_seed(4))
     yp = _host(linear.matmul(tx[..., perm.to(tx.device), :].contiguous(), tw, ts), m)
@@ -109,21 +139,29 @@ def test_epilogue(device, fmt, m, k, n):
     tw, h = _weight(device, n, k, fmt, 11)
     x, tx = _x(device, m, k, 12)
     want = O.ref(x, h)
+    exact, err = _products(tx, h)
     res = torch.randn(m, n, generator=torch.Generator().manual_seed(13)).to(torch.bfloat16)
     tr = res.reshape(1, 1, m, n).to(device.torch)
+    plus, err_plus = exact + tr[0, 0].double(), err + tr[0, 0].double().abs() * 2.0**-23
     for mode in ("epilogue", "preload"):
-        y = _host(linear.matmul(tx, tw, None, residual=tr, residual_mode=mode), m)
-        check(f"residual {mode}", y, want + res.float())
-        y = _host(linear.matmul(tx, tw, None, residual=tr, residual_mode=mode, out32=True), m)
-        check(f"residual {mode} fp32", y, want + res.float(), rel=1e-3, pcc=0.999999)
+        yd = linear.matmul(tx, tw, None, residual=tr, residual_mode=mode)
+        check(f"residual {mode}", _host(yd, m), want + res.float())
+        _near(f"residual {mode}, every value", yd, plus, err_plus)
+        yd = linear.matmul(tx, tw, None, residual=tr, residual_mode=mode, out32=True)
+        check(f"residual {mode} fp32", _host(yd, m), want + res.float(), rel=1e-3, pcc=0.999999)
+        _near(f"residual {mode} fp32, every value", yd, plus, err_plus)
     inplace = tr.clone()
     assert linear.matmul(tx, tw, None, residual=inplace, out=inplace) is inplace
     check("residual in place", _host(inplace, m), want + res.float())
-    check("fp32 output", _host(linear.matmul(tx, tw, None, out32=True), m), want, rel=1e-3, pcc=0.999999)
+    _near("residual in place, every value", inplace, plus, err_plus)
+    yd = linear.matmul(tx, tw, None, out32=True)
+    check("fp32 output", _host(yd, m), want, rel=1e-3, pcc=0.999999)
+    _near("fp32 output, every value", yd, exact, err)
     wide = torch.full((1, 1, m, 32 + n + 32), 7.0, dtype=torch.bfloat16, device=device.torch)
     linear.matmul(tx, tw, None, out=wide, col0=1)
     y = _host(wide, m)
     check("col0", y[:, 32:32 + n], want)
+    _near("col0, every value", wide.reshape(m, -1)[:, 32:32 + n], exact, err)
     rest = torch.cat([y[:, :32], y[:, 32 + n:]], 1)
     same("the other columns untouched", rest, torch.full_like(rest, 7.0))
 
@@ -143,9 +181,12 @@ def test_glu(device, fmt, m, k, n):
                               dtype=linear.float32)
     xd = x.to(torch.bfloat16).double()
     g, u = (xd @ hg.double()) * s[0].double(), (xd @ hu.double()) * s[1].double()
+    (gx, ge), (ux, ue) = ([v * sc.to(tx.device).double() for v in _products(tx, h)] for h, sc in ((hg, s[0]), (hu, s[1])))
     for act, code in (("swiglu", 0), ("geglu", 1)):
-        two = _host(linear.matmul(tx, tg, tsg, glu=True, w_up=tu, scale_up=tsu, glu_act=code), m)
+        yd = linear.matmul(tx, tg, tsg, glu=True, w_up=tu, scale_up=tsu, glu_act=code)
+        two = _host(yd, m)
         check(f"{fmt} {act} two weights", two, O.glu_ref(g, u, act))
+        _near(f"{act}, every value", yd, *_glu(gx, ge, ux, ue, act))
         same("interleaved against two weights", _host(linear.matmul(tx, ti, tsi, glu=True, glu_act=code), m), two)
 
 
@@ -176,23 +217,34 @@ def test_glu_float32(device, fmt, m, k, n):
     tg, tu = (linear.native_weight(device, w, FMTS[fmt])[0] for w in (gw, uw))
     x, tx = _x(device, m, k, 53)
     xd = x.to(torch.bfloat16).double().to(device.torch)
-    y = _host(linear.matmul(tx, tg, None, glu=True, w_up=tu, out32=True), m)
-    check(f"{fmt} swiglu float32", y, O.glu_ref((xd @ hg).cpu(), (xd @ hu).cpu(), "swiglu"), rel=1e-5, pcc=0.999999)
+    yd = linear.matmul(tx, tg, None, glu=True, w_up=tu, out32=True)
+    check(f"{fmt} swiglu float32", _host(yd, m), O.glu_ref((xd @ hg).cpu(), (xd @ hu).cpu(), "swiglu"), rel=1e-5, pcc=0.999999)
+    _near("every value", yd, *_glu(*_products(tx, hg), *_products(tx, hu), "swiglu"))
 
 
 @pytest.mark.gpu
-def test_columns_past_k_and_nan(device):
+@pytest.mark.parametrize("fmt", list(FMTS))
+@pytest.mark.parametrize("m, k, n, glu", [(140, 288, 64, False), (131, 288, 14340, False), (70, 1056, 7200, True),
+                                          (333, 96, 8224, True)])
+def test_columns_past_k_and_nan(device, fmt, m, k, n, glu):
     """A ragged K: what lies past K in x's memory (the next row, here Inf and NaN) enters no sum; a NaN row stays its
-    own row's."""
-    m, k, n = 140, 288, 64
-    tw, h = _weight(device, n, k, "bfp8", 31)
+    own row's. In tiles whose wavefronts split K and in those that share x, each format's order of k, a GLU, and a float32
+    y's."""
+    tw, h = _weight(device, n, k, fmt, 31)
+    tu, hu = _weight(device, n, k, fmt, 33) if glu else (None, None)
     x, _ = _x(device, m, k, 32)
-    x[5] = float("nan")
-    x[7, 3] = float("inf")
-    y = _host(linear.matmul(x.to(torch.bfloat16).reshape(1, 1, m, k).to(device.torch), tw, None), m)
-    assert bool(y[5].isnan().all()) and not bool(y[7].isfinite().any())
-    keep = [r for r in range(m) if r not in (5, 7)]
-    check("the other rows", y[keep], O.ref(x[keep], h))
+    rows = [5, m - 2]  # (NaN; the row after each has an Inf)
+    x[rows] = float("nan")
+    x[[r + 1 for r in rows], 3] = float("inf")
+    tx = x.to(torch.bfloat16).reshape(1, 1, m, k).to(device.torch)
+    keep = torch.tensor([r for r in range(m) if r not in rows and r - 1 not in rows], device=device.torch)
+    kept = tx[..., keep, :]
+    want = _products(kept, h) if not glu else _glu(*_products(kept, h), *_products(kept, hu), "swiglu")
+    for out32 in (False, True):
+        y = linear.matmul(tx, tw, None, out32=out32, **({"glu": True, "w_up": tu} if glu else {})).reshape(m, -1)
+        for r in rows:
+            assert bool(y[r].isnan().all()) and not bool(y[r + 1].isfinite().any())
+        _near(f"{fmt} K {k} N {n} {y.dtype}: the other rows", y[keep], *want)
 
 
 def test_staging_order():

@@ -10,7 +10,7 @@ bound carried through the activation."""
 import pytest
 import torch
 
-from common.testing import same
+from common.testing import same, within
 from moe import moe8
 from oracle import dense_oracle as O
 from oracle import moe_oracle as MO
@@ -58,6 +58,48 @@ def test_down_rows(device, E, k, H, I, R):
     bound = ref.abs() * 2.0 ** -8 + mag * (len(u) * I * 2.0 ** -24) + 1e-30
     assert bool((err <= bound).all()), f"worst {float((err / bound).max()):.3f} of its bound"
     assert not yd[R:].any(), "rows past R"
+
+
+# What lies past the chosen experts' columns of h (here NaN), or past a row's last ones (the next row, here NaN), enters no
+# sum, at an expert's K of a part of a step: both kernels of the down, the one of up to 16 rows, and the K-block one. The
+# bound is test_down_rows'.
+@pytest.mark.parametrize("E, k, H, I, R, kblock", [
+    (16, 4, 4128, 288, 32, False),  # pairs
+    (4, 4, 8224, 160, 17, False),  # pairs, one split
+    (4, 2, 64, 160, 24, False),  # one
+    (16, 2, 2080, 480, 18, False),  # one, several splits
+    (16, 4, 1056, 288, 9, False),
+    (4, 2, 64, 160, 24, True),
+])
+@pytest.mark.parametrize("all_chosen", [False, True])
+def test_down_nan_beside(device, E, k, H, I, R, kblock, all_chosen):
+    print(f"case E {E} k {k} H {H} I {I} rows {R} kblock {kblock} all {all_chosen}", flush=True)
+    g = torch.Generator().manual_seed(H + I)
+
+    def grid(w):
+        return torch.from_numpy(MO.held_kblock(w.numpy()) if kblock else O.held(w, "bfp4")).float()
+
+    dn = torch.stack([grid(torch.randn(I, H, generator=g) * 0.05) for _ in range(E)])
+    P = moe8.pack(device, torch.zeros(E, H, 2 * I, dtype=BF), dn.to(BF), kblock=kblock)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(R)])
+    if all_chosen:
+        ids = (torch.arange(R * k) % E).reshape(R, k)
+    else:
+        ids[:] = ids[0]
+    tid = ids.to(torch.int16).reshape(1, 1, R, k).to(device.torch)
+    u = sorted(set(ids.flatten().tolist()))
+    units = min(E, R * k)
+    assert (len(u) == units) == all_chosen or k == E
+    h = torch.randn(32, units * I, generator=g).to(BF)
+    h[:, len(u) * I:] = float("nan")
+    h[R - 2] = float("nan")
+    y = moe8.down_rows(h.reshape(1, 1, 32, units * I).to(device.torch), P, tid, k, R)
+    yd = y.reshape(-1, y.shape[-1])[:R, :H]
+    assert bool(yd[R - 2].isnan().all())
+    keep = [r for r in range(R) if r != R - 2]
+    hd, wt = h[keep, :len(u) * I].double(), torch.cat([dn[e] for e in u]).double()
+    ref, mag = hd @ wt, hd.abs() @ wt.abs()
+    within("the other rows", yd[keep].cpu(), ref, ref.abs() * 2.0 ** -8 + mag * (len(u) * I * 2.0 ** -24) + 1e-30)
 
 
 # more workgroups than one round of 8 wavefronts takes: 4 wavefronts of one run of K each (6 and 9 groups of 256 k:
