@@ -181,26 +181,27 @@ int dr_topk_merge(const void* records, int n_records, int rows, int k, int fp32,
 /* The work split for K and M: chunks (waves per output tile, each a K range of kch values) and the rows a pass
  * takes (M picks the kernel: the GEMV for 1-2 rows, the MFMA kernel from 3, whose chunks are 256 k up to K = 3072
  * against the GEMV's up to 2048). For inspection of block-float and bf16 weights (dr_launch_plan
- * gives any launch's own plan, an int4 weight's and that of more than 128 rows among them); results depend only on what this returns. */
+ * gives any launch's own plan, an int4 weight's and the tiled kernel's of many rows among them). */
 int dr_plan(int k, int m, int32_t* chunks, int32_t* kch, int32_t* rows_per_pass);
 
 /* What dr_matmul would launch for this launch, for inspection (replaces the plan dict that dense_reader/linear.py:
  * 455-495 choose/plan return): the kernel, the output tile width, the work split and the top-k records it writes. */
 typedef struct dr_launch_info {
     int32_t kernel;        /* 0: the VALU GEMV (rows <= 2, int4 <= 5), 1: an MFMA kernel */
-    int32_t rows_per_pass; /* (from 129 rows on one launch takes all rows: its workgroups' rows, 64 to 256) */
+    int32_t rows_per_pass; /* (one launch of the tiled kernel, from 129 rows, a GLU's 33, on: its workgroups' rows, 64
+                              to 256) */
     int32_t tile_cols;     /* output columns of a work tile: 16 (one panel) or 32 */
     int32_t tiles;         /* work tiles of the launch */
     int32_t chunks;        /* K chunks a tile, kch values each */
     int32_t kch;
     int32_t splits;        /* workgroups a tile (split K), 1 if unsplit */
     int32_t workgroups;    /* workgroups of one pass */
-    int32_t passes;        /* row passes: launches, or (from 129 rows on) the row tiles of the one launch */
+    int32_t passes;        /* row passes: launches, or the row tiles of the tiled kernel's one */
     int32_t records;       /* top-k records the launch writes (0: no top-k) */
     int32_t tiles_per_record;
     int32_t waves;         /* wavefronts a workgroup (each walks its K chunks in turn) */
     int32_t tiles_per_workgroup; /* 2: a 32-row launch of more tiles than CUs, its block-float segments' tiles in
-                                    pairs (bf16 segments one a workgroup); from 129 rows on 8 or 2 (a GLU's 4 or 1);
+                                    pairs (bf16 segments one a workgroup); the tiled kernel's 8 or 2 (a GLU's 4 or 1);
                                     else 1 */
     int32_t lds_bytes;     /* LDS a workgroup of the first pass's kernel, static and dynamic (0 without a device) */
     int32_t reserved[2];

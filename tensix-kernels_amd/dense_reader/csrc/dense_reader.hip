@@ -58,7 +58,6 @@ __host__ __device__ constexpr int tile_w() {
     return PW == 1 ? 16 : TILE;
 }
 
-
 // DR_BFP4_KB: the byte of a panel's exponents that holds column c's exponent for k (one a 16-k group): per 128-k block
 // 128 bytes, lane (kq, c) of the block's wavefront load at 2 (16 kq + c), its two groups (k 32 kq + 0..15, + 16..31)
 __host__ __device__ constexpr int exp_off_kb(int k, int c) {
@@ -78,7 +77,6 @@ typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a), __builtin_bit_cast(bf16x2, b), c, false);
 }
-
 
 struct Args {
     const uint16_t* x;
@@ -700,7 +698,6 @@ __device__ __forceinline__ void chunk_bf16(const Args& a, const uint8_t* const* 
     }
 }
 
-
 // The epilogue's operands from memory (column scales, residual), read before the K loop so that their latency hides
 // under it instead of adding to the workgroup's end: thread c < TW (the tile's width) the scales of the tile's output
 // column c (gate and up with a GLU), thread e the residual of its first epilogue element (row e / TW, column e % TW).
@@ -750,7 +747,6 @@ __device__ __forceinline__ void epi_stage(const EpiPre& p, float* pre) {
     }
     pre[PRE_RES + e] = p.res;
 }
-
 
 // the experts' act(g) * u: act_glu's two, or swiglu_oai min(g, 7) * sigmoid(1.702 min(g, 7)) * (clamp(u, -7, 7) + 1)
 // (dense_ops.h:90-118), a NaN passing through the clamps as it does there (the dense GLU keeps act_glu alone: the
@@ -1087,8 +1083,9 @@ __device__ __forceinline__ void epilogue(const Args& a, const SegDev& sg, int t,
 // panels then as many up panels: 32 columns, or 16 in a narrow launch (PW = 2).
 // The rows' routing weights come from cw (moe_coefs) where the kernel found them before its K loop, else from here; a
 // thread's elements are all of one column, whose bias is read once, before the sums.
-// run: the sums that part's are added to ([PW][ROWS][16]; null: zeros).
-template <int ROWS, int PW, int MOE>
+// run: the sums that part's are added to (null: zeros). LANES (32 rows): part and run are [PW][2][64 lanes][4], each lane's
+// four rows of a 16-row block as the MFMA leaves them, instead of [PW][ROWS][16].
+template <int ROWS, int PW, int MOE, bool LANES = false>
 __device__ __forceinline__ void epilogue_moe(const MoeArgs& a, int t, int unit, int ex, const float* part, int nparts,
                                              float wunit, const uint32_t* cw = nullptr,
                                              const float* run = nullptr) {
@@ -1121,7 +1118,9 @@ __device__ __forceinline__ void epilogue_moe(const MoeArgs& a, int t, int unit, 
     for (int e = threadIdx.x; e < TW * ROWS; e += wg_threads(a)) {
         const int m = e / TW;
         if (m >= mrows || oc >= a.en) continue;
-        const int cq = col >> 4, cc = col & 15, ig = (cq * ROWS + m) * 16 + cc, iu = ((H + cq) * ROWS + m) * 16 + cc;
+        const int cq = col >> 4, cc = col & 15;
+        const int at = LANES ? ((m >> 4) * 64 + ((m & 15) >> 2) * 16 + cc) * 4 + (m & 3) : m * 16 + cc;
+        const int ig = cq * ROWS * 16 + at, iu = (H + cq) * ROWS * 16 + at;
         float gsum = sum_parts(run != nullptr ? run[ig] : 0.f, part + ig, nparts, PW * ROWS * 16);
         float usum = sum_parts(run != nullptr ? run[iu] : 0.f, part + iu, nparts, PW * ROWS * 16);
         if (a.bias != nullptr) {
@@ -1366,7 +1365,6 @@ __global__ __launch_bounds__(512) void dr_gemv_g1(const Args a) {
     gemv_body<MR, PW, FMT, ONE, true, PLAIN>(a);
 }
 
-
 // ---- the expert gather (include/moe.h): the GEMV and MFMA kernels over the chosen experts' bfloat4_b weights ----------
 //
 // Kernels of their own (the dense kernels stay as they are: a gather branch in them, even compiled out, moved the
@@ -1529,7 +1527,6 @@ dr_gemv_moe(const MoeArgs a) {
 // block-float m * 2^(E - bias) (exact in bf16: at most 7 significant bits), the power of two broadcast across the row
 // from the lane that read that k's exponent. Output lane l: rows 4 (l / 16) .. +3 of column l % 16.
 
-
 // d = broadcast(s from lane I of this row of 16) * f (the same hazard rule as fmac_bcast)
 template <int I, bool NOP>
 __device__ __forceinline__ float mul_bcast(float s, float f) {
@@ -1542,7 +1539,6 @@ __device__ __forceinline__ float mul_bcast(float s, float f) {
                      : "=v"(d) : "v"(s), "v"(f), "i"(I));
     return d;
 }
-
 
 // 16 bytes of x: row m, columns k .. k + 7 (k a multiple of 8). Rows past x read its last row: they only reach output
 // rows that are never written. Columns past K read its last columns and are zeroed by x_kmask (the weights there are
@@ -1611,7 +1607,6 @@ template <int NCH>
 __device__ __forceinline__ uint4 x_lds(const uint4* xs, int row, int c) {
     return xs[NCH * row + (c ^ x_swz<NCH>(row))];
 }
-
 
 // B for 8 bfp8 values: bytes 8H .. 8H + 7 of the lane's codes (k-offsets 16 kq + 8H + j), times the broadcast scales
 template <int H>
@@ -2620,6 +2615,7 @@ template <int NT, bool TWO>
 __device__ __forceinline__ void moe_pair_tiles(const MoeArgs& a, int t0, int unit, int ex, int wave, int lane,
                                                float* part, const uint32_t* cw) {
     constexpr int PW = 4 * NT, ROWS = 32;
+    constexpr int E = 4 * ROWS * 16;  // a tile's sums
     const SegDev& sg = a.seg[0];
     const uint8_t* cb[PW];
     const uint8_t* eb[PW];
@@ -2642,18 +2638,14 @@ __device__ __forceinline__ void moe_pair_tiles(const MoeArgs& a, int t0, int uni
             for (int tt = 0; tt < 2; ++tt) acc[q][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
     auto store = [&](float* to, int u) {  // tile u's sums of this wavefront
-        const int l = (int)opaque((uint32_t)lane);  // (addresses made here, not held across the K loop)
+        f32x4* t = reinterpret_cast<f32x4*>(to) + wave * (E / 4) + opaque((uint32_t)lane);  // (not held across the K loop)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    to[((wave * 4 + q) * ROWS + 16 * tt + 4 * (l >> 4) + j) * 16 + (l & 15)] = acc[4 * u + q][tt][j];
+            for (int tt = 0; tt < 2; ++tt) t[(2 * q + tt) * 64] = acc[4 * u + q][tt];
     };
     clear();
     uint4* xs = reinterpret_cast<uint4*>(part) + wave * (XS_BYTES / 16);
-    constexpr int E = 4 * ROWS * 16;  // a tile's sums
     float* meet = part + 4 * (XS_BYTES / 4);  // TWO: a tile's sums of each wavefront, and the first of two tiles' total
     int nparts = a.waves;
     if constexpr (TWO) {
@@ -2680,9 +2672,15 @@ __device__ __forceinline__ void moe_pair_tiles(const MoeArgs& a, int t0, int uni
                     lds_barrier();
                     float* to = meet + (NT == 2 && u == 0 ? 4 * E : 0);
 #pragma unroll
-                    for (int i = 0; i < E / 256; ++i) {
-                        const int e = threadIdx.x + 256 * i;
-                        to[e] = sum_parts(0.f, meet + e, 4, E);
+                    for (int i = 0; i < E / 1024; ++i) {
+                        const int e = 4 * (threadIdx.x + 256 * i);
+                        f32x4 v[4];
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) v[w] = *reinterpret_cast<const f32x4*>(meet + w * E + e);
+                        f32x4 sum;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) sum[j] = 0.f + v[0][j] + v[1][j] + v[2][j] + v[3][j];
+                        *reinterpret_cast<f32x4*>(to + e) = sum;
                     }
                 }
                 clear();
@@ -2699,7 +2697,7 @@ __device__ __forceinline__ void moe_pair_tiles(const MoeArgs& a, int t0, int uni
         __syncthreads();  // (the staging, or the previous tile's epilogue, done with part)
         store(part, u);
         __syncthreads();
-        epilogue_moe<ROWS, 4, DR_MOE_GATE_UP_ROWS>(a, t0 + u, unit, ex, part, nparts, 0.f, cw,
+        epilogue_moe<ROWS, 4, DR_MOE_GATE_UP_ROWS, true>(a, t0 + u, unit, ex, part, nparts, 0.f, cw,
                                                     !TWO ? nullptr : meet + (NT == 2 && u == 0 ? 4 * E : 0));
     }
 }
@@ -2727,8 +2725,9 @@ __global__ __launch_bounds__(TWO ? 256 : 512, 2) void dr_mfma_moe_pairs(const Mo
 // DR_MOE_DOWN_ROWS at 32 rows: two adjacent 32-column tiles a workgroup (the last of an odd count alone), so that the
 // staged x serves both, and the union's steps (its experts' K one after another) shared out evenly over the splits'
 // wavefronts, each one run of them. With a chunk of 512 k at a time over one tile, each wavefront had 2 KB of codes in
-// flight and started cold at every chunk: the gpt-oss shape at 17 and 32 rows took 78 and 86 us, and takes 59 and 64 now
-// (132.7 MB of codes: 2.2 and 2.1 TB/s, the decoding's rate). LDS: the wavefronts' x staging, then the partial sums of
+// flight and started cold at every chunk: the gpt-oss shape at 17 and 32 rows takes 74 and 91 us so, 57 and 66 here
+// (132.7 MB of codes at 32: 2.0 TB/s, the decoding's rate; down_in_pairs says which shapes take which). Of its 128
+// registers 3 are spilled before the K loop and read back after it. LDS: the wavefronts' x staging, then the partial sums of
 // the second tile, which meet first, and of the first.
 __global__ __launch_bounds__(512, 4) void dr_mfma_moe_down_pairs(const MoeArgs a) {
     extern __shared__ float part[];
@@ -3713,8 +3712,8 @@ void bind_split(Args& a, void* workspace, int pw, int mr) {
 // 37, 44, 180 -> 14 (the call's host time). Up to 128 rows the passes stay: their rows equal those of a call on them
 // alone bit for bit.
 // A GLU's passes are 16 rows, and it goes over from 33 rows on (a block list's single calls, up to 32 rows, keep the
-// passes' sums): bfloat8_b gate
-// and up K = 4096 N = 14336 at 33, 64 and 128 rows 78, 107, 215 -> 45, 45, 51 us, bfloat4_b 58, 78, 157 -> 41, 42, 50.
+// passes' sums): bfloat8_b gate and up K = 4096 N = 14336 at 33, 64 and 128 rows 78, 107, 215 -> 45, 45, 51 us,
+// bfloat4_b 58, 78, 157 -> 41, 42, 50. Where the passes are faster they stay (gemm_plan).
 constexpr int GEMM_MIN_M = 129, GEMM_MIN_M_GLU = 33;
 
 // The tile: mt row tiles of 32 with the wavefronts side by side (256 columns a workgroup, 128 with a GLU), or ks, 64
@@ -3886,7 +3885,6 @@ void* scratch_for_stream(hipStream_t st, int& status) {
     }
     return scratch_addr[cur];
 }
-
 
 }  // namespace
 
@@ -4246,17 +4244,17 @@ int prepare_moe(const dr_launch* L, const dr_moe* M, MoeArgs& a, int& pw, int& t
     }
     limit_splits(a);
     a.chains = a.waves;
-    // The MFMA rows of gate/up, more workgroups than one round and a tenth of 8 wavefronts each (two on a CU at 16 rows,
-    // one at 32, by registers; those of the chosen experts count, the others end at once): 4 wavefronts of two chains of
-    // chunks each, so that one workgroup's start and epilogue pass under another's K loop. 12 chunks over 8 wavefronts
-    // left half of them idle for half of it too. The chains and their order are those of a wavefront each, so a row's
-    // bits do not depend on the choice. (The gpt-oss gate/up at 3, 8, 16, 17 and 32 rows 40, 65, 88, 110, 134 us in 8
-    // wavefronts, 36, 55, 76, 89, 111 in 4; over 365 shapes past the line 4 are 15 % faster at the mean and 4 % slower at
-    // the most, in the 80 between one round of all experts and the line up to 16 % slower: 32 experts of top 1, 768 columns,
-    // K = 2304, 32 rows 24.1 against 28.0.)
+    // The MFMA rows of gate/up, more workgroups than one round of 8 wavefronts each (two on a CU at 16 rows, one at 32, by
+    // registers; those of the chosen experts count, the others end at once), a tenth more at 16 rows and eight chunks or
+    // more, which leave fewer wavefronts idle: 4 wavefronts of two chains of chunks each, so that one workgroup's start and
+    // epilogue pass under another's K loop. 12 chunks over 8 wavefronts left half of them idle for half of it too. The
+    // chains and their order are those of a wavefront each, so a row's bits do not depend on the choice. (The gpt-oss
+    // gate/up at 3, 8, 16, 17 and 32 rows 40, 65, 88, 110, 134 us in 8 wavefronts, 36, 55, 76, 87, 107 in 4; over 365
+    // shapes past the line 4 are 15 % faster at the mean and 4 % slower at the most, in the 80 between one round of all
+    // experts and the line up to 16 % slower: 32 experts of top 1, 768 columns, K = 2304, 32 rows 24.1 against 28.0.)
     if (nmode && mr >= 16 && a.splits == 1 && a.waves > 4) {
         const int te = mr == 32 && s0.fmt == DR_BFP4 ? (a.tpe + 1) / 2 : a.tpe;
-        if (chosen * te > (mr == 32 ? 1.1 : 2.2) * cu_count()) a.waves = 4;
+        if (chosen * te > (mr == 32 ? 1. : a.chunks < 8 ? 2. : 2.2) * cu_count()) a.waves = 4;
     }
     return DR_OK;
 }
