@@ -284,9 +284,10 @@ def reference(x, w, scale=None):
 def row_slices(x, full_sync=False):
     """[(first tile row, tile rows)] of x's rows, at most 4 tile rows each (8 with full_sync) (reference linear.py:
     179-184, where each slice is one program that reads all the weights). matmul needs no slicing: one call takes all of
-    x's rows, up to 128 of them in passes of plan()["rows_per_pass"], more in one launch of a tiled kernel. A caller that slices x this way gets each slice's
-    rows from its own matmul (the rows a call takes pick its kernel, so the sums of a slice's rows can differ in their
-    last bits from those of one call over all rows)."""
+    x's rows, up to 128 of them (a GLU's 32) in passes of plan()["rows_per_pass"], more in one launch of a tiled kernel
+    (or, where that is faster, in passes too). A caller that slices x this way gets each slice's rows from its own matmul
+    (the rows a call takes pick its kernel, so the sums of a slice's rows can differ in their last bits from those of one
+    call over all rows)."""
     mt = -(-x.shape[-2] // TILE)
     cap = 8 if full_sync else 4
     return [(m0, min(cap, mt - m0)) for m0 in range(0, mt, cap)]

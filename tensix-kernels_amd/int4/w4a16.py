@@ -109,7 +109,8 @@ def w4a16_linear(x, wq, scale, *, memory_config=None, fidelity="hifi2", **opts):
 
 def rows_matmul(x2, wq, scale):
     """y [M, N] bf16 = x2 [M, K] (bf16, GPU) @ (q * s).T: dr_matmul with a DR_INT4 segment, any M (up to 5 rows on
-    the GEMV, each row's result that of a one-token call; more on the MFMA kernel, 16 or 32 a pass)."""
+    the GEMV, each row's result bit for bit that of a one-token call; more on the MFMA kernel, 16 or 32 a pass, whose
+    sums run in another order: equal to rounding)."""
     L, y, x2 = _launch(x2, wq, scale)
     linear.run(L, x2.device, "dr_matmul (int4)")
     return y
