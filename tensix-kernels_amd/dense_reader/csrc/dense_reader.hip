@@ -4106,14 +4106,19 @@ int down_pair_splits(const MoeArgs& a, int units, int tiles) {
     return std::max(1, std::min({2 * cu_count() / tp, DOWN_SPLITS, (most + MAXW - 1) / MAXW}));
 }
 
+// the one-tile kernel's split sums, which its last workgroup gathers, at most (the CU's LDS less what it holds besides)
+constexpr int DOWN_LDS = 144 << 10;
+
 // Whether the down of 17 to 32 rows takes less time in tile pairs than a tile a workgroup (a holds that plan). Both
 // times in us, as fitted to 356 shapes on MI355X (8 to 64 experts, H 256 to 4096, I 128 to 2880, 17 and 32 rows; within
 // 7 and 3 % of the measured ones at the mean): a workgroup's start and end, the splits' meeting, then the steps of 128 k
 // of its wavefronts, with one workgroup on a CU and with more. The pairs keep every CU busy for the whole of K at the
 // larger shapes (H = I = 2880, 32 experts: 91 -> 66 us), but cost more where a wavefront has few steps or their few
 // splits leave CUs idle (H = 1536, I = 768, 17 rows of top 1: 16.3 against 22.6; H = 512, I = 2048, 64 experts: 31 and
-// 46). A float32 y stays with the one-tile kernel, whose wavefronts sum at most 1024 k each. Over the 356, the choice is up to 4 % slower than the one-tile kernel alone and 5 % faster at the mean.
+// 46). A float32 y stays with the one-tile kernel, whose wavefronts sum at most 1024 k each. Over the 356, the choice is
+// up to 4 % slower than the one-tile kernel alone and 5 % faster at the mean.
 bool down_in_pairs(const MoeArgs& a, double chosen, int tiles, int pair_splits) {
+    if ((int64_t)a.splits * 2 * 32 * 16 * 4 > DOWN_LDS) return true;
     const double cus = cu_count(), steps = chosen * ((a.ek + 127) / 128);
     const int per = (a.cps + MAXW - 1) / MAXW * a.kch / 128;  // a wavefront's steps
     const double wgs = tiles * std::max(1., chosen * a.ekp / a.kch / a.cps);

@@ -33,6 +33,7 @@ BF = torch.bfloat16
     (16, 4, 4128, 288, 18),  # pairs: 4 experts chosen of the 16 expected
     (4, 4, 8224, 160, 17),  # pairs: one split
     (8, 4, 1024, 768, 32),  # one: every wavefront two chunks of 256 k
+    (256, 8, 64, 1408, 32),  # pairs: the 48 splits' sums of the one-tile kernel would not fit the LDS
 ])
 def test_down_rows(device, E, k, H, I, R):
     print(f"case E {E} k {k} H {H} I {I} rows {R}", flush=True)
