@@ -6,6 +6,7 @@
 namespace drk {
 
 constexpr int GEMM_W = 4;  // wavefronts a workgroup, side by side over the columns
+constexpr int F32_MT4_K = 4096;
 
 struct GemmArgs {
     const uint16_t* x;
@@ -21,7 +22,7 @@ struct GemmArgs {
     SegDev seg;
 };
 
-// mt: row tiles of 32 a workgroup (2, 4, 6 or 8; 2 for a float32 y); ks: the wavefronts split K (mt 2)
+// mt: row tiles of 32 a workgroup (2, 4, 6 or 8; for a float32 y 2, or 4 of block-float up to K = F32_MT4_K); ks: the wavefronts split K (mt 2)
 hipError_t launch_gemm(const GemmArgs& g, int mt, bool ks, hipStream_t st);
 
 // LDS bytes a workgroup: four stages of x, 64 k of its rows each (ks: one for each wavefront)

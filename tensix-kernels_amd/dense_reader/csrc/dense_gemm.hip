@@ -85,10 +85,14 @@ struct StepCodes {
 // MT row tiles of 32, two column tiles of 32 a wavefront (with GLU the gate's and the up's). KS: the wavefronts split
 // K instead of lying side by side. acc: lane l's sums, row 32 t + l % 32, columns 8 g + 4 (l / 32) + 0 .. 3 of tile n in
 // words 4 g + 0 .. 3.
-// F32 (a float32 y, which shows the sums' rounding): the accumulators hold 256 k at a time, added up in three levels of
-// eight. One accumulator for all of K rounds at each of its K / 16 MFMAs, which at K = 4096 and 14336 was 2.5 and
-// 4.5 times the error of the passes of 32 rows (bfloat8_b 2.0e-7 against 8.0e-8, 4.7e-7 against 1.04e-7); so it is no
-// larger than theirs (7.4e-8, 8.7e-8; measured at K = 96 to 28672, each format).
+// F32 (a float32 y, which shows the sums' rounding): the accumulators are carried over into further sums before they grow
+// long. One accumulator for all of K rounds at each of its K / 16 MFMAs, which at K = 4096 and 14336 was 2.5 and 4.5 times
+// the error of the passes of 32 rows (bfloat8_b 2.0e-7 against 8.0e-8, 4.7e-7 against 1.04e-7). At 64 rows they hold 256 k
+// at a time, added up in three levels of eight; at 128 (block-float, up to K = F32_MT4_K), where the registers leave room for
+// one more sum of each (bfloat8_b: but for two, kept in scratch), 256 k up to K = 2048 and 512 past it, added up in turn,
+// much as the passes' wavefronts do. No larger an error than the passes' at any K (7.4e-8, 8.7e-8; measured at K = 96 to
+// 28672, each format). 1000 rows K = 4096 N = 14336 444 us in passes, 126 with one accumulator, 235 in tiles of 64 rows,
+// 168 of 128.
 template <int MT, int FMT, bool GLU, bool KS, bool F32>
 __device__ __forceinline__ void gemm_k_loop(const GemmArgs& a, int nt, int m0, f32x16 (&acc)[2][MT], uint4* x0, uint4* x1,
                                             uint4* x2, uint4* x3) {
@@ -97,7 +101,7 @@ __device__ __forceinline__ void gemm_k_loop(const GemmArgs& a, int nt, int m0, f
     constexpr int NX = 32 * MT * 8 / (64 * XW);                // 16-byte x chunks a lane stages a step
     constexpr int NC = FMT == DR_BFP8 ? 2 : FMT == DR_BFP4 ? 1 : 4;
     constexpr int NG = 4 * MT;                                 // groups of two MFMAs a step
-    constexpr int PF = 3;                                      // x operands read ahead
+    constexpr int PF = F32 && MT > 2 ? 1 : 3;                  // x operands read ahead (fewer where registers are short)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, p = (lane >> 4) & 1, h = lane >> 5;
     const int t0 = KS ? nt * OT : (nt * GEMM_W + wave) * OT;   // the wavefront's first output tile
@@ -230,12 +234,15 @@ __device__ __forceinline__ void gemm_k_loop(const GemmArgs& a, int nt, int m0, f
         if constexpr (q == 3) B[n][u].w = w;
     };
 
-    f32x16 l1[2][F32 ? MT : 1], l2[2][F32 ? MT : 1], l3[2][F32 ? MT : 1];  // sums of 256, 2048 and 16384 k
+    constexpr int L = !F32 ? 0 : MT == 2 ? 3 : 1;  // sums beside the accumulators
+    f32x16 lev[L ? L : 1][2][L ? MT : 1];            // (L 3: of 256, 2048 and 16384 k)
     if constexpr (F32) {
 #pragma unroll
-        for (int n = 0; n < 2; ++n)
+        for (int l = 0; l < L; ++l)
 #pragma unroll
-            for (int t = 0; t < MT; ++t) l1[n][t] = l2[n][t] = l3[n][t] = acc[n][t];  // (zeros)
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) lev[l][n][t] = acc[n][t];  // (zeros)
     }
     StepCodes<FMT> k0, k1, k2, k3;  // step s's codes in k[s % 4], asked for three steps ahead
     uint4 B0[2][4], B1[2][4];       // the decoded operands of even and odd steps (bf16 weights: the codes themselves)
@@ -325,16 +332,23 @@ __device__ __forceinline__ void gemm_k_loop(const GemmArgs& a, int nt, int m0, f
                         for (int i = 0; i < 16; ++i) from[n][t][i] = 0.f;
                     }
             };
-            carry(l1, acc);
-            if (((g - g0) & 7) == 7) carry(l2, l1);
-            if (((g - g0) & 63) == 63) carry(l3, l2);
+            if constexpr (L == 1) {
+                if (a.k_pad <= 2048 || ((g - g0) & 1)) carry(lev[0], acc);
+            } else {
+                carry(lev[0], acc);
+                if (((g - g0) & 7) == 7) carry(lev[1], lev[0]);
+                if (((g - g0) & 63) == 63) carry(lev[2], lev[1]);
+            }
         }
     }
     if constexpr (F32) {
 #pragma unroll
         for (int n = 0; n < 2; ++n)
 #pragma unroll
-            for (int t = 0; t < MT; ++t) acc[n][t] = l3[n][t] + l2[n][t] + l1[n][t];
+            for (int t = 0; t < MT; ++t) {
+                if constexpr (L == 1) acc[n][t] = lev[0][n][t] + acc[n][t];
+                else acc[n][t] = lev[2][n][t] + lev[1][n][t] + lev[0][n][t];
+            }
     }
 }
 
@@ -508,6 +522,7 @@ template <int MT, bool KS, bool F32>
 void launch_gemm_t(const GemmArgs& g, hipStream_t st) {
     const dim3 grid(g.tm * g.tn), b(64 * GEMM_W);
     const bool glu = g.seg.glu != 0;
+    constexpr bool BF16 = !F32 || MT == 2;  // (gemm_plan's tiles)
     switch (g.seg.fmt) {
         case DR_BFP8:
             if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BFP8, true, KS, F32>), grid, b, 0, st, g);
@@ -518,8 +533,10 @@ void launch_gemm_t(const GemmArgs& g, hipStream_t st) {
             else hipLaunchKernelGGL((dr_gemm<MT, DR_BFP4, false, KS, F32>), grid, b, 0, st, g);
             break;
         default:
-            if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BF16, true, KS, F32>), grid, b, 0, st, g);
-            else hipLaunchKernelGGL((dr_gemm<MT, DR_BF16, false, KS, F32>), grid, b, 0, st, g);
+            if constexpr (BF16) {
+                if (glu) hipLaunchKernelGGL((dr_gemm<MT, DR_BF16, true, KS, F32>), grid, b, 0, st, g);
+                else hipLaunchKernelGGL((dr_gemm<MT, DR_BF16, false, KS, F32>), grid, b, 0, st, g);
+            }
             break;
     }
 }
@@ -527,7 +544,8 @@ void launch_gemm_t(const GemmArgs& g, hipStream_t st) {
 }  // namespace
 
 hipError_t launch_gemm(const GemmArgs& g, int mt, bool ks, hipStream_t st) {
-    if (g.y_f32) ks ? launch_gemm_t<2, true, true>(g, st) : launch_gemm_t<2, false, true>(g, st);
+    if (g.y_f32 && mt == 4) launch_gemm_t<4, false, true>(g, st);
+    else if (g.y_f32) ks ? launch_gemm_t<2, true, true>(g, st) : launch_gemm_t<2, false, true>(g, st);
     else if (ks) launch_gemm_t<2, true, false>(g, st);
     else if (mt == 8) launch_gemm_t<8, false, false>(g, st);
     else if (mt == 6) launch_gemm_t<6, false, false>(g, st);

@@ -3727,8 +3727,9 @@ struct GemmTile {
     int start, step;
 };
 constexpr GemmTile GEMM_TILES[] = {{2, true, 100, 28}, {2, false, 300, 66}, {4, false, 500, 86}, {6, false, 700, 111}, {8, false, 900, 139}};
-// a float32 y: a round of ks 9, 21 and 66 us at K = 1024, 4096 and 14336, of 64 rows 21, 65 and 193 (dense_gemm.hip's F32)
-constexpr GemmTile GEMM_TILES_F32[] = {{2, true, 400, 28}, {2, false, 700, 80}};
+// a float32 y: a round of ks 9, 21 and 66 us at K = 1024, 4096 and 14336, of 64 rows 24, 64 and 193, of 128 37 and 88
+// (dense_gemm.hip's F32)
+constexpr GemmTile GEMM_TILES_F32[] = {{2, true, 400, 28}, {2, false, 1100, 82}, {4, false, 2000, 106}};
 
 // The passes' time in the same unit: each pass a start and end, the splits' meeting and, for each round of workgroups
 // over the CUs, a wavefront's k (1024 of them 12.6 us, bf16's 16; of a GLU's two weights 13 and 22). A last pass of at
@@ -3770,6 +3771,7 @@ bool gemm_plan(const dr_launch* L, const Args& a, int pw, int mr, GemmArgs& g, G
     const GemmTile* tiles = a.y_f32 ? GEMM_TILES_F32 : GEMM_TILES;
     for (size_t i = 0; i < (a.y_f32 ? std::size(GEMM_TILES_F32) : std::size(GEMM_TILES)); ++i) {
         const GemmTile& t = tiles[i];
+        if (a.y_f32 && t.mt == 4 && (a.k > F32_MT4_K || s.fmt == DR_BF16)) continue;
         const int per = (s.glu ? 1 : 2) * (t.ks ? 1 : GEMM_W);  // output tiles a workgroup
         const long long tm = (a.m + 32 * t.mt - 1) / (32 * t.mt), tn = (g.tiles + per - 1) / per;
         const long long rounds = (tm * tn + cu_count() - 1) / cu_count();

@@ -195,8 +195,8 @@ def test_split_k_meeting_order(library_asm):
 
 
 def scratch_in_mfma_loops(asm):
-    """[(function, scratch instructions)] of the innermost loops that hold both a matrix instruction and an access to
-    scratch memory: registers spilled inside a K loop."""
+    """[(function, scratch instructions)] of the innermost loops that hold a matrix instruction and more than one access to
+    scratch memory in 500 lines: registers spilled inside a K loop."""
     found = []
     for name, body in re.findall(r"^(_Z\S+):(.*?)^\.Lfunc_end", asm, re.M | re.S):
         lines = [s.split(";")[0].strip() for s in body.split("\n")]
@@ -207,7 +207,7 @@ def scratch_in_mfma_loops(asm):
             if any((b, e) != (b2, e2) and b <= b2 and e2 <= e for b2, e2 in loops):
                 continue
             n = sum(s.startswith("scratch_") for s in lines[b:e])
-            if n and any(s.startswith("v_mfma") for s in lines[b:e]):
+            if 500 * n > e - b and any(s.startswith("v_mfma") for s in lines[b:e]):
                 found.append((name, n))
     return found
 
