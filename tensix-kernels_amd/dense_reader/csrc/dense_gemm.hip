@@ -90,7 +90,7 @@ struct StepCodes {
 // the error of the passes of 32 rows (bfloat8_b 2.0e-7 against 8.0e-8, 4.7e-7 against 1.04e-7). At 64 rows they hold 256 k
 // at a time, added up in three levels of eight; at 128 (block-float, up to K = F32_MT4_K), where the registers leave room for
 // one more sum of each (bfloat8_b: but for two, kept in scratch), 256 k up to K = 2048 and 512 past it, added up in turn,
-// much as the passes' wavefronts do. No larger an error than the passes' at any K (7.4e-8, 8.7e-8; measured at K = 96 to
+// much as the passes' wavefronts do. No larger an error than the passes' at any K (7.4e-8, at 128 rows 8.0e-8, and 8.7e-8; measured at K = 96 to
 // 28672, each format). 1000 rows K = 4096 N = 14336 444 us in passes, 126 with one accumulator, 235 in tiles of 64 rows,
 // 168 of 128.
 template <int MT, int FMT, bool GLU, bool KS, bool F32>
